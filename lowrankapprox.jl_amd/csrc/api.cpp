@@ -443,6 +443,7 @@ extern "C" int lra_geqp3_adap_f64(lra_ctx* c, int64_t m, int64_t n, double* B, i
   q.nb = (int)std::min<i64>(nb, std::max<i64>(kmax, 1));
   q.mode = 0; q.atol = atol; q.rtol = rtol; q.jpvt = jpvt; q.tau = tau; q.vn1 = nullptr;
   q.vn2 = nullptr; q.stop_after = 0; q.k_out = dk; q.early_out = nullptr;
+  q.exact_tail = 1;
   LRA_CHECK(lra_qrcp(c, q));
   i64 hk = 0;
   LRA_CHECK(read_scalars(c, dk, &hk, 1));

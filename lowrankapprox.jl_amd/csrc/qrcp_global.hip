@@ -3,8 +3,9 @@
 // kernel of qrcp.hip (e.g. order 1032 or 2056 on thousands of columns).
 //
 // The sketch stays in HBM (column-major, in place).  Up to 8192 rows (with the uncached
-// exchange area) each pivot step is ONE launch, `qg_fused` (below): every workgroup rebuilds
-// the step's reflector itself, and the workgroup that finishes last picks the next pivot.
+// exchange area) the steps run in blocks of up to 16 (qrcp_block.hip), and where blocks come out
+// short each step is ONE launch, `qg_fused` (below): every workgroup rebuilds the step's
+// reflector itself, and the workgroup that finishes last picks the next pivot.
 // Otherwise (or with LRA_QG_FUSED=0) each step is two launches on the context's stream, with
 // every decision kept on the device:
 //   qg_step   one workgroup: dlaqps block bookkeeping and the stop rule for the step just
@@ -16,7 +17,7 @@
 //             test gets its norm recomputed and ends the block.
 // Once the stop rule fires, the remaining launches return at once.  The arithmetic and the
 // control follow qrcp_kernel, so both give the same pivots up to rounding.
-#include "lra_internal.h"
+#include "lra_qg.h"
 #include "lra_wave.h"
 
 #include <algorithm>
@@ -454,11 +455,6 @@ __global__ void qg_finish(const GState* st, i64* k_out, int* early_out) {
 // that a co-resident cooperative grid kept from being dispatched.)  Workgroup 0 stores v(s), tau(s) and R(s,s); the pivot column itself is
 // rewritten one launch later, when no workgroup reads it any more.
 
-struct FState {
-  int j0, jb, done, k, early, sprev, pad0, pad1;
-  double ptol;
-};
-
 typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 
 // The exchange area of the fused steps: kSubCtr + 1 ticket counters kCtrStride words apart
@@ -511,6 +507,11 @@ __global__ __launch_bounds__(GT) void qg_fstart(int n, int kmax, int nb, const d
     st->jb = min(nb, kmax);
     st->early = 0;
     st->sprev = -1;
+    st->s = 0;
+    st->b = 0;
+    st->mask = 0;
+    st->ncand = 0;
+    st->tau = -1.0;
     int done = kmax <= 0 ? 1 : 0;
     st->k = kmax > 0 ? kmax : 0;
     if (!done && (cp < 0 || cp >= n)) {  // no candidate (NaN norms)
@@ -631,6 +632,7 @@ LRA_DEV void fused_finish(int s, int n, int kmax, int nb, int stop_after, double
     allok &= tok[q];
   }
   st->sprev = s;
+  st->s = s + 1;
   if (!allok) {  // a partial never landed: stop with an error
     __hip_atomic_store(err, LRA_E_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     st->k = s + 1;
@@ -679,7 +681,7 @@ LRA_DEV void fused_finish(int s, int n, int kmax, int nb, int stop_after, double
 
 // one fused step s; NWC waves per column, RPL rows per lane (rows s..m-1 fit 64 NWC RPL)
 template <int NWC, int RPL>
-__global__ __launch_bounds__(256) void qg_fused(int s, int m, int n, int kmax, int nb,
+__global__ __launch_bounds__(256) void qg_fused(int s, int s_first, int m, int n, int kmax, int nb,
                                                 int stop_after, int lastrk,
                                                 double* __restrict__ B, i64 ldb, int* at,
                                                 double* vn1, double* vn2, double* tau,
@@ -756,7 +758,7 @@ __global__ __launch_bounds__(256) void qg_fused(int s, int m, int n, int kmax, i
       tau[s] = tu;
       diag[s] = beta;
     }
-    if (s > 0) {
+    if (s > s_first) {  // (columns of steps before s_first are whole)
       const double* vp = vbuf + (size_t)((s - 1) & 1) * m;
       double* d = B + (i64)at[s - 1] * ldb;
       for (int t = s - 1 + tid; t < m; t += 256) d[t] = t == s - 1 ? diag[s - 1] : vp[t];
@@ -1369,12 +1371,12 @@ int lra_zqrcp_global(lra_ctx* c, double* Bz, i64 ldb, int m, int n, int kmax, in
 namespace {
 
 // the fused launch of step s: rows s..m-1 (at most 8192) pick the form, as for the applies
-void launch_fused(hipStream_t s0, int s, const QrcpCall& q, int lastrk, int* at, double* vn1,
+void launch_fused(hipStream_t s0, int s, int s_first, const QrcpCall& q, int lastrk, int* at, double* vn1,
                   double* vn2, double* diag, double* vbuf, FState* st, u64x2* part,
                   unsigned* ctr, int* err) {
   const int m = q.m, n = q.n, rows = m - s, tr = n - s - 1;
   auto grid = [&](int cpb) { return dim3((unsigned)std::max(1, (tr + cpb - 1) / cpb)); };
-#define QF_ARGS s, m, n, q.kmax, q.nb, q.stop_after, lastrk, q.A, q.lda, at, vn1, vn2, q.tau, \
+#define QF_ARGS s, s_first, m, n, q.kmax, q.nb, q.stop_after, lastrk, q.A, q.lda, at, vn1, vn2, q.tau, \
                 diag, vbuf, st, part, ctr, err
   if (rows <= 64 * 8)
     hipLaunchKernelGGL((qg_fused<1, 8>), grid(4), dim3(256), 0, s0, QF_ARGS);
@@ -1439,16 +1441,59 @@ int lra_qrcp_global(lra_ctx* c, const QrcpCall& q) {
       hipLaunchKernelGGL(qg_fstart, dim3(1), dim3(GT), 0, s0, n, q.kmax, q.nb, vn1, q.atol,
                          q.rtol, fs, at);
       LRA_HIP(hipGetLastError());
-      for (int s = 0; s < q.kmax; ++s) {
-        launch_fused(s0, s, q, lastrk, at, vn1, vn2, diag, v, fs, part, ctr, c->d_err);
-        LRA_HIP(hipGetLastError());
-        if ((s & 63) == 63) {  // stop enqueueing once the device has stopped
-          int done = 0;
-          LRA_HIP(hipMemcpyAsync(c->host_pinned, &fs->done, sizeof(int), hipMemcpyDeviceToHost,
-                                 s0));
-          LRA_HIP(hipStreamSynchronize(s0));
-          std::memcpy(&done, c->host_pinned, sizeof(int));
-          if (done) break;
+      auto read_state = [&](FState* h) -> int {
+        LRA_HIP(hipMemcpyAsync(c->host_pinned, fs, sizeof(FState), hipMemcpyDeviceToHost, s0));
+        LRA_HIP(hipStreamSynchronize(s0));
+        std::memcpy(h, c->host_pinned, sizeof(FState));
+        return LRA_OK;
+      };
+      FState h{};
+      // single steps first .. first + count - 1 (stopping early once the device has stopped)
+      auto single = [&](int first, int count) -> int {
+        const int last = std::min(q.kmax, first + count);
+        for (int s = first; s < last; ++s) {
+          launch_fused(s0, s, first, q, lastrk, at, vn1, vn2, diag, v, fs, part, ctr, c->d_err);
+          LRA_HIP(hipGetLastError());
+          if ((s & 63) == 63 && s + 1 < last) {
+            LRA_CHECK(read_state(&h));
+            if (h.done) break;
+          }
+        }
+        return LRA_OK;
+      };
+      // Blocks of steps where their workspace fits the budget (LRA_QG_BLOCK=0: single steps
+      // only).  A block takes 57 to 92 us (rows 900 to 2056, 3758 columns) against 10 to 24 us
+      // for a single step, about four of them, so where the blocks come out shorter than
+      // kShort steps on average (many columns of nearly equal norm, or norms outside the
+      // blocks' range) single steps run, twice as many each time.
+      const char* be = getenv("LRA_QG_BLOCK");
+      double* wb = nullptr;
+      const bool block = !(be && be[0] == '0') && lra_wsT(c, WS_QGB, lra_qb_doubles(m), &wb) == LRA_OK;
+      if (!block) {
+        LRA_CHECK(single(0, q.kmax));
+      } else {
+        const QbWork w = lra_qb_work(wb, m);
+        constexpr int kBatch = 8, kShort = 3;
+        LRA_CHECK(lra_qb_start(c, q, w, at, vn1, diag, fs));
+        for (int s = 0, run = 64;;) {
+          LRA_CHECK(lra_qb_blocks(c, q, w, at, vn1, vn2, diag, fs, s, kBatch));
+          LRA_CHECK(read_state(&h));
+          const int steps = h.s - s;
+          s = h.s;
+          if (h.done) break;
+          if (steps >= kShort * kBatch) {
+            run = 64;
+            continue;
+          }
+          LRA_CHECK(lra_qb_pick(c, w, at, fs));
+          LRA_CHECK(single(s, run));
+          hipLaunchKernelGGL(qg_ffinish, dim3(1), dim3(256), 0, s0, m, q.A, q.lda, at, diag, v, fs,
+                             q.k_out, q.early_out);
+          LRA_CHECK(lra_qb_start(c, q, w, at, vn1, diag, fs));
+          LRA_CHECK(read_state(&h));
+          s = h.s;
+          if (h.done) break;
+          run = std::min(2 * run, 4096);
         }
       }
       hipLaunchKernelGGL(qg_ffinish, dim3(1), dim3(256), 0, s0, m, q.A, q.lda, at, diag, v, fs,

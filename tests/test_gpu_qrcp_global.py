@@ -143,3 +143,97 @@ def test_slow_decay_orders_1032_to_2600(gpu, orc):
     e_o = np.linalg.norm(A[:, V_o.rd - 1] - A[:, V_o.sk - 1] @ V_o.T, 2)
     assert e_g <= 10 * max(e_o, 1e-15)
     assert e_g <= 1e3 * 1e-10
+
+
+def _edge_matrix(kind, m, n, seed):
+    rng = np.random.default_rng(seed)
+    B = graded(m, n, seed, decay=0.99)
+    if kind == "ties":          # every column of the same norm, many exactly equal
+        B = np.asfortranarray(np.tile(rng.standard_normal((m, 4)), (1, (n + 3) // 4))[:, :n])
+    elif kind == "lowrank":     # rank 37 exactly: zero residuals after 37 steps
+        B = np.asfortranarray(rng.standard_normal((m, 37)) @ rng.standard_normal((37, n)))
+    elif kind == "zeros":       # zero columns among the others
+        B[:, ::3] = 0.0
+    elif kind == "cliff":       # columns whose norm falls by 1e6 within a block
+        u = rng.standard_normal((m, 5))
+        B = np.asfortranarray(u @ rng.standard_normal((5, n)) + 1e-6 * rng.standard_normal((m, n)))
+    elif kind == "huge":        # outside the range of the blocks: single steps
+        B = np.asfortranarray(B * 1e148)
+    elif kind == "tiny":
+        B = np.asfortranarray(B * 1e-148)
+    elif kind == "slow":        # 16-step blocks, norms recomputed (early dlaqps block ends)
+        U, _ = np.linalg.qr(rng.standard_normal((m, min(m, n))))
+        V, _ = np.linalg.qr(rng.standard_normal((n, min(m, n))))
+        B = np.asfortranarray((U * np.exp(-0.03 * np.arange(min(m, n)))) @ V.T)
+    elif kind == "steep":       # the pivots' own norms fall far enough to end dlaqps blocks
+        U, _ = np.linalg.qr(rng.standard_normal((m, min(m, n))))
+        V, _ = np.linalg.qr(rng.standard_normal((n, min(m, n))))
+        B = np.asfortranarray((U * np.exp(-0.3 * np.arange(min(m, n)))) @ V.T)
+    return B
+
+
+@pytest.mark.parametrize("kind,m,n,rtol,rank", [
+    ("graded", 40, 9, 0.0, -1), ("graded", 17, 300, 0.0, -1), ("slow", 700, 500, 1e-13, -1),
+    ("slow", 1040, 700, 1e-9, -1), ("slow", 2100, 333, 1e-7, 200), ("slow", 3100, 260, 1e-7, -1),
+    ("slow", 5000, 140, 0.0, 77), ("slow", 530, 1300, 1e-8, 33), ("ties", 200, 600, 0.0, 40),
+    ("lowrank", 300, 700, 1e-10, -1), ("zeros", 300, 301, 1e-9, -1), ("cliff", 400, 640, 1e-9, -1),
+    ("steep", 100, 60, 1e-8, -1), ("steep", 64, 200, 1e-7, -1), ("steep", 90, 75, 1e-9, -1),
+    ("steep", 1100, 81, 1e-8, -1), ("huge", 300, 400, 1e-8, -1), ("tiny", 300, 400, 1e-8, -1)])
+def test_blocks_match_single_steps(gpu, monkeypatch, kind, m, n, rtol, rank):
+    """Blocks of steps against one launch per step on the same matrix: the same rank and pivots,
+    all n positions (the columns past the rank included), R and the reflectors to rounding times
+    the condition of their step.  Where columns tie or have no residual left, any order is a
+    pivoted QR: there the product Q R is compared with the permuted matrix instead."""
+    import torch
+    monkeypatch.setenv("LRA_QRCP_GLOBAL", "1")
+    B = _edge_matrix(kind, m, n, m + 5 * n)
+    out = {}
+    for block in ("1", "0"):
+        monkeypatch.setenv("LRA_QG_BLOCK", block)
+        print(f"blocks {kind} m={m} n={n} rtol={rtol} rank={rank} block={block}", flush=True)
+        Bd = gpu.to_device(B).clone().t().contiguous().t()
+        p, tau, k = gpu.geqp3_adap(Bd, rank, 0.0, rtol, 32)
+        torch.cuda.synchronize()
+        out[block] = (host(p), host(tau), k, host(Bd))
+    (p1, t1, k1, B1), (p0, t0, k0, B0) = out["1"], out["0"]
+    assert k1 == k0
+    if kind in ("ties", "lowrank", "cliff"):
+        assert np.array_equal(np.sort(p1), np.arange(1, n + 1))
+        kk = k1
+        V = np.tril(B1[:, :kk], -1) + np.eye(m, kk)
+        X = np.zeros((m, n))
+        X[:kk] = np.triu(B1[:kk])
+        for j in range(kk - 1, -1, -1):
+            X -= t1[j] * np.outer(V[:, j], V[:, j] @ X)
+        E = X - B[:, p1 - 1]
+        d = np.abs(np.diag(B1)[:kk])
+        assert (d[1:] <= d[:-1] * (1 + 1e-7)).all()  # (the downdated norms' accuracy)
+        tail = max(rtol * d[0] * np.sqrt(n * max(1, min(m, n) - kk)), 1e-12 * d[0])
+        rest = 0.0 if kk < min(m, n) and rank >= 0 else np.linalg.norm(E[:, kk:], axis=0).max()
+        assert np.abs(E[:, :kk]).max() <= 1e-12 * d[0] and rest <= 10 * tail
+        return
+    assert np.array_equal(p1, p0)
+    kk = min(k1, m, n)
+    scale = np.abs(B0[:kk]).max()
+    assert np.abs(np.triu(B1[:kk]) - np.triu(B0[:kk])).max() <= 1e-11 * scale
+    cond = np.abs(B0[0, 0]) / np.abs(np.diag(B0[:kk, :kk]))
+    dv = np.abs(np.tril(B1[:, :kk], -1) - np.tril(B0[:, :kk], -1)).max(axis=0)
+    assert np.all(dv <= 1e-12 * cond), int(np.argmax(dv / cond))
+    assert np.all(np.abs(t1[:kk] - t0[:kk]) <= 1e-12 * cond)
+
+
+def test_blocks_nan_column(gpu, monkeypatch):
+    """A NaN column is never a pivot, in either form, and the others are factored alike."""
+    import torch
+    monkeypatch.setenv("LRA_QRCP_GLOBAL", "1")
+    B = _edge_matrix("slow", 400, 300, 3)
+    B[7, 11] = np.nan
+    got = []
+    for block in ("1", "0"):
+        monkeypatch.setenv("LRA_QG_BLOCK", block)
+        Bd = gpu.to_device(B).clone().t().contiguous().t()
+        p, _, k = gpu.geqp3_adap(Bd, 60, 0.0, 1e-9, 32)
+        torch.cuda.synchronize()
+        got.append((host(p), k))
+    assert got[0][1] == got[1][1] == 60
+    assert np.array_equal(got[0][0][:60], got[1][0][:60]) and 12 not in got[0][0][:60]
