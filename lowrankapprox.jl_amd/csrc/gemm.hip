@@ -417,6 +417,112 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
     }
 }
 
+// C (M x N <= 16 NT) = alpha op(A) op(B) + beta C, FP64, one 32-row tile and one K range per
+// workgroup; each wave takes every fourth 16-deep step of the range and the four partial tiles
+// meet in LDS.  Operands go from memory to the MFMA registers: with k = 4 q + r for register r of
+// lane quarter q, a lane reads four consecutive k of a k-contiguous operand (32 bytes), or one row
+// of 16 lanes each of four k of an m-contiguous one (128 bytes).  A is read once; B (at most 64
+// columns) comes from L1/L2.  The next step's operands load during the current step's MFMAs.
+// Bound by the MFMAs and the reading of A in turn: 64 columns on 8192 x 436 (m-contiguous) take
+// 24 us a call (213 by the tiled kernel), on 436 x 7756 with beta = 1 32 us (215), on their
+// transposes 35 (43) and 30 us (132); 16 columns 17, 21, 20 and 16 us.
+typedef double d2a8 __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int TA, int TB, int NT>
+__global__ __launch_bounds__(256) void gemm_narrow_kernel(
+    int M, int N, int K, int kchunk, const double* __restrict__ A, i64 lda,
+    const double* __restrict__ B, i64 ldb, double* __restrict__ part, double alpha, double beta,
+    double* __restrict__ C, i64 ldc) {
+  __shared__ double red[4][32][16 * NT + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, q = lane >> 4;
+  const int m0 = (int)blockIdx.x * 32, n0 = (int)blockIdx.z * 16 * NT;
+  const int k0 = (int)blockIdx.y * kchunk, k1 = min(K, k0 + kchunk);
+  const double* pa[2];
+  const double* pb[NT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const i64 m = min(m0 + 16 * i + l16, M - 1);
+    pa[i] = TA ? A + m * lda : A + m;
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const i64 n = min(n0 + 16 * j + l16, N - 1);
+    pb[j] = TB ? B + n : B + n * ldb;
+  }
+  auto load4 = [&](const double* p, int contiguous, i64 ld, int k, double* v) {
+    if (k + 16 - 4 * q <= k1) {  // the whole step is in range (the same for every lane)
+      if (contiguous) {
+        const d2a8 a = *reinterpret_cast<const d2a8*>(p + k);
+        const d2a8 b = *reinterpret_cast<const d2a8*>(p + k + 2);
+        v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = p[(i64)(k + r) * ld];
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const i64 kk = min(k + r, k1 - 1);
+        const double x = p[contiguous ? kk : kk * ld];
+        v[r] = k + r < k1 ? x : 0.0;
+      }
+    }
+  };
+  double a[2][4], b[NT][4];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) load4(pa[i], TA, lda, k + 4 * q, a[i]);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) load4(pb[j], !TB, ldb, k + 4 * q, b[j]);
+  };
+  d4 acc[2][NT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = d4{0, 0, 0, 0};
+  int k = k0 + 16 * wave;
+  if (k < k1) load(k);
+  for (; k < k1; k += 64) {
+    double ca[2][4], cb[NT][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) ca[i][r] = a[i][r];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) cb[j][r] = b[j][r];
+    }
+    if (k + 64 < k1) load(k + 64);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[i][r], cb[j][r], acc[i][j], 0, 0, 0);
+  }
+  // register r holds row q + 4 r of its tile
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave][16 * i + q + 4 * r][16 * j + l16] = acc[i][j][r];
+  __syncthreads();
+  for (int e = tid; e < 32 * 16 * NT; e += 256) {
+    const int row = e & 31, cl = e >> 5, col = n0 + cl;
+    const i64 m = m0 + row;
+    if (m >= M || col >= N) continue;
+    const double v = (red[0][row][cl] + red[1][row][cl]) + (red[2][row][cl] + red[3][row][cl]);
+    if (part) {
+      part[(i64)blockIdx.y * M * N + m + (i64)col * M] = v;
+    } else {
+      double* c = C + m + (i64)col * ldc;
+      *c = beta == 0.0 ? alpha * v : alpha * v + beta * *c;
+    }
+  }
+}
+
 __global__ void splitk_reduce_kernel(int M, int N, int splits, const double* part, double alpha,
                                      double beta, double* C, i64 ldc) {
   const i64 total = (i64)M * N;
@@ -761,6 +867,56 @@ int run_tn_skinny(lra_ctx* ctx, const GemmArgs& g) {
   return LRA_OK;
 }
 
+// op(A) op(B) with few columns (a factor applied to a block of vectors) on gemm_narrow_kernel:
+// 32 x 64 tiles whose four waves share K, K split further over workgroups (chunks of at least
+// 128) until about two workgroups per CU run.  One pass over op(A) for every 64 columns, no LDS
+// staging: the tiled kernels' 128-column tiles spend half or more of their MFMAs on padding, run
+// on a few CUs (8192 x 436 by 64 columns: 64 workgroups) and are not tuned with beta != 0.
+// Where the line lies (times of a call, tiled -> narrow): an operand that is not k-contiguous is
+// read by narrow in any case up to 256 columns (8192 x 436: 224 -> 56 us at 256 columns, 8192 x
+// 2048: 263 -> 201); with both k-contiguous the tuned tiles read it from LDS as well, and beyond
+// 64 columns narrow is ahead only for short K (7756 x 436 at 128 columns 143 -> 48 us, 200 x
+// 2000 34 -> 16, but 4096 x 4096 105 -> 121).
+bool narrow_ok(const GemmArgs& g) {
+  if (g.prec != LRA_PREC_F64 || g.bgather != nullptr || g.K < 1 || g.N > 256) return false;
+  return g.N <= 64 || g.K <= 2048 || !kc_ok(g);
+}
+
+int run_narrow(lra_ctx* ctx, const GemmArgs& g) {
+  const i64 mt = (g.M + 31) / 32, nt = (g.N + 63) / 64, tiles = mt * nt;
+  i64 splits = std::max<i64>(1, std::min<i64>((2 * ctx->num_cu + tiles - 1) / tiles, g.K / 128));
+  i64 kchunk = (g.K + splits - 1) / splits;
+  kchunk = (kchunk + 63) / 64 * 64;
+  splits = (g.K + kchunk - 1) / kchunk;
+  double* part = nullptr;
+  if (splits > 1) LRA_CHECK(lra_wsT(ctx, WS_SPLITK, (size_t)(splits * g.M * g.N), &part));
+  const dim3 grid((unsigned)mt, (unsigned)splits, (unsigned)nt);
+#define NARROW(TA, TB, NT)                                                                     \
+  hipLaunchKernelGGL((gemm_narrow_kernel<TA, TB, NT>), grid, dim3(256), 0, ctx->stream,        \
+                     (int)g.M, (int)g.N, (int)g.K, (int)kchunk, g.A, g.lda, g.B, g.ldb, part,  \
+                     g.alpha, g.beta, g.C, g.ldc)
+#define NARROW_T(NT)                                                                           \
+  if (g.transA) { if (g.transB) NARROW(1, 1, NT); else NARROW(1, 0, NT); }                     \
+  else { if (g.transB) NARROW(0, 1, NT); else NARROW(0, 0, NT); }
+  if (g.N <= 16) { NARROW_T(1) }
+  else if (g.N <= 32) { NARROW_T(2) }
+  else { NARROW_T(4) }
+#undef NARROW_T
+#undef NARROW
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && splits > 1) {
+    const int rb = (int)std::min<i64>((g.M * g.N + 255) / 256, 16384);
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(rb), dim3(256), 0, ctx->stream, (int)g.M,
+                       (int)g.N, (int)splits, part, g.alpha, g.beta, g.C, g.ldc);
+    e = hipGetLastError();
+  }
+  if (e != hipSuccess) {
+    lra_set_error("narrow gemm launch: %s", hipGetErrorString(e));
+    return LRA_E_HIP;
+  }
+  return LRA_OK;
+}
+
 void candidates(const GemmArgs& g, int num_cu, std::vector<TuneVal>* out) {
   const bool kc = kc_ok(g);
   for (int cfg = 0; cfg < kNumCfg; ++cfg) {
@@ -841,6 +997,7 @@ int lra_gemm(lra_ctx* ctx, const GemmArgs& g) {
   }
   if (tn_skinny_ok(g)) return run_tn_skinny(ctx, g);
   if (ct_ok(g)) return run_ct(ctx, g);
+  if (narrow_ok(g)) return run_narrow(ctx, g);
   TuneKey key{g.prec, g.transA, g.transB, bucket_m(g.M), bucket(g.N), bucket(g.K)};
   TuneVal choice;
   bool have = false;

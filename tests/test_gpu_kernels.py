@@ -268,3 +268,29 @@ def test_sketch_gemm_f32_kc_configs(gpu, monkeypatch, cfg, M, N, K):
     ref = Om @ A
     err = np.abs(B - ref).max() / np.sqrt(K)
     assert err < 2e-5, err
+
+
+@pytest.mark.parametrize("ta", ["n", "c"])
+@pytest.mark.parametrize("tb", ["n", "c"])
+@pytest.mark.parametrize("M,N,K,beta", [
+    (1, 1, 1, 0.0), (31, 16, 15, 0.5), (32, 17, 16, 0.0), (33, 64, 65, -2.0), (300, 65, 129, 0.0),
+    (65, 1, 4099, 0.0), (129, 256, 1000, 1.0), (20, 33, 8192, 1.0), (2049, 5, 63, 0.0),
+    (70, 130, 2049, 0.0)])
+def test_dgemm_narrow(gpu, ta, tb, M, N, K, beta):
+    """Products with few columns, every storage order, odd offsets and leading dimensions, against
+    float64 numpy: sums of K terms in any order differ by at most K eps |a||b| a term."""
+    rng = np.random.default_rng(M + 3 * N + K)
+    import torch
+
+    def stored(r, c):
+        big = torch.from_numpy(rng.standard_normal((c, r + 5))).cuda()
+        return big[:, 3:3 + r].t()  # ld r + 5, base 8 bytes off a 16-byte boundary
+
+    A = stored(K, M) if ta == "c" else stored(M, K)
+    B = stored(N, K) if tb == "c" else stored(K, N)
+    C = stored(M, N)
+    Ah, Bh, Ch = host(A), host(B), host(C).copy()
+    Ah, Bh = (Ah.T if ta == "c" else Ah), (Bh.T if tb == "c" else Bh)
+    gpu.dgemm(A, B, ta, tb, 1.5, C, beta)
+    bound = 2.3e-16 * (K + 4) * (1.5 * np.abs(Ah) @ np.abs(Bh) + np.abs(beta * Ch))
+    assert (np.abs(host(C) - (1.5 * Ah @ Bh + beta * Ch)) <= bound).all()
