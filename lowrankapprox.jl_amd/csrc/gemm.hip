@@ -272,9 +272,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmDev p) {
 
 // FP64 GEMM for the case where both operands are k-contiguous in memory (op(A) = A' with A
 // stored K x M, op(B) = B stored K x N, no gather): the sketch B = Omega * A.  Every thread
-// moves 16-byte pairs (two consecutive k) from HBM into registers for the next k-tile while
-// the MFMAs consume the current one from a second LDS buffer, so each k-tile costs one
-// barrier.  LDS rows hold BK = 16 doubles padded to 17, which keeps the 16 lanes of an MFMA
+// moves 16-byte pairs (two consecutive k) from HBM into registers two k-tiles ahead of the
+// MFMAs, which consume the current one from one of two LDS buffers, so each k-tile costs one
+// (LDS-only) barrier.  LDS rows hold BK = 16 doubles padded to 17, which keeps the 16 lanes of an MFMA
 // operand read on distinct banks.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BK = 16, bool F32 = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(GemmDev p) {
@@ -305,53 +305,59 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
   typedef double d2 __attribute__((ext_vector_type(2)));
-  d2 ra[LA], rb[LB];
-  // chunk e of a tile -> (row e / KP, k pair e % KP)
-  auto load_tiles = [&](int k0) {
+  // chunk e of a tile -> (row e / KP, k pair e % KP).  Rows past M (columns past N) are read from
+  // the last one, and chunks past the tile from its last: unconditional loads, so the wait for
+  // one tile's registers leaves the loads of the next in flight.  What they put in the tile
+  // reaches only outputs that are not stored.
+  const double *pa[LA], *pb[LB];
+  int oa[LA], ob[LB];
 #pragma unroll
-    for (int t = 0; t < LA; ++t) {
-      const int e = tid + NT * t;
-      const int r = e / KP, c = (e % KP) * 2;
-      const int gm = m0 + r, gk = k0 + c;
-      d2 v = {0.0, 0.0};
-      if (e < CA && gm < p.M) {
-        const double* src = p.A + gk + (i64)gm * p.lda;
-        if (gk + 1 < kend) v = *reinterpret_cast<const d2*>(src);
-        else if (gk < kend) v.x = src[0];
-      }
-      ra[t] = v;
-    }
+  for (int t = 0; t < LA; ++t) {
+    const int e = min(tid + NT * t, CA - 1), r = e / KP, c = (e % KP) * 2;
+    pa[t] = p.A + kbeg + c + (i64)min(m0 + r, p.M - 1) * p.lda;
+    oa[t] = r * LDK + c;
+  }
 #pragma unroll
-    for (int t = 0; t < LB; ++t) {
-      const int e = tid + NT * t;
-      const int r = e / KP, c = (e % KP) * 2;
-      const int gn = n0 + r, gk = k0 + c;
-      d2 v = {0.0, 0.0};
-      if (e < CB && gn < p.N) {
-        const double* src = p.B + gk + (i64)gn * p.ldb;
-        if (gk + 1 < kend) v = *reinterpret_cast<const d2*>(src);
-        else if (gk < kend) v.x = src[0];
-      }
-      rb[t] = v;
-    }
+  for (int t = 0; t < LB; ++t) {
+    const int e = min(tid + NT * t, CB - 1), r = e / KP, c = (e % KP) * 2;
+    pb[t] = p.B + kbeg + c + (i64)min(n0 + r, p.N - 1) * p.ldb;
+    ob[t] = r * LDK + c;
+  }
+  auto load_tiles = [&](d2 (&ra)[LA], d2 (&rb)[LB], int tile) {
+    const i64 o = (i64)tile * BK;
+#pragma unroll
+    for (int t = 0; t < LA; ++t) ra[t] = *reinterpret_cast<const d2*>(pa[t] + o);
+#pragma unroll
+    for (int t = 0; t < LB; ++t) rb[t] = *reinterpret_cast<const d2*>(pb[t] + o);
   };
-  auto store_tiles = [&](int buf) {
+  // the last tile when the range does not end on one: k beyond the range is zero
+  auto load_tail = [&](d2 (&ra)[LA], d2 (&rb)[LB], int tile) {
+    const int left = kend - kbeg - tile * BK;
+    const i64 o = (i64)tile * BK;
+    auto get = [&](const double* src, int c) {
+      d2 v = {0.0, 0.0};
+      if (c + 1 < left) v = *reinterpret_cast<const d2*>(src);
+      else if (c < left) v.x = src[0];
+      return v;
+    };
+#pragma unroll
+    for (int t = 0; t < LA; ++t) ra[t] = get(pa[t] + o, oa[t] % LDK);
+#pragma unroll
+    for (int t = 0; t < LB; ++t) rb[t] = get(pb[t] + o, ob[t] % LDK);
+  };
+  auto store_tiles = [&](const d2 (&ra)[LA], const d2 (&rb)[LB], int buf) {
 #pragma unroll
     for (int t = 0; t < LA; ++t) {
-      const int e = tid + NT * t;
-      if (e < CA) {
-        const int o = (e / KP) * LDK + (e % KP) * 2;
-        sA[buf][o] = (E)ra[t].x;
-        sA[buf][o + 1] = (E)ra[t].y;
+      if (CA % NT == 0 || tid + NT * t < CA) {
+        sA[buf][oa[t]] = (E)ra[t].x;
+        sA[buf][oa[t] + 1] = (E)ra[t].y;
       }
     }
 #pragma unroll
     for (int t = 0; t < LB; ++t) {
-      const int e = tid + NT * t;
-      if (e < CB) {
-        const int o = (e / KP) * LDK + (e % KP) * 2;
-        sB[buf][o] = (E)rb[t].x;
-        sB[buf][o + 1] = (E)rb[t].y;
+      if (CB % NT == 0 || tid + NT * t < CB) {
+        sB[buf][ob[t]] = (E)rb[t].x;
+        sB[buf][ob[t] + 1] = (E)rb[t].y;
       }
     }
   };
@@ -363,37 +369,87 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
     for (int j = 0; j < TN; ++j) acc[i][j] = ACC{0, 0, 0, 0};
   const int l16 = lane & 15, lq = lane >> 4;
   const int am0 = wm * WTM, bn0 = wn * WTN;
-
-  // (the pointer alignment of the 16-byte loads: lda, ldb, kchunk and k0 are even)
-  if (kbeg < kend) {
-    load_tiles(kbeg);
-    store_tiles(0);
-    __syncthreads();
-    int cur = 0;
-    for (int k0 = kbeg; k0 < kend; k0 += BK) {
-      const bool more = k0 + BK < kend;
-      if (more) load_tiles(k0 + BK);
+  auto compute = [&](int buf) {
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        E af[TM], bfv[TN];
+    for (int kk = 0; kk < BK; kk += 4) {
+      E af[TM], bfv[TN];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) af[i] = sA[cur][(am0 + i * 16 + l16) * LDK + kk + lq];
+      for (int i = 0; i < TM; ++i) af[i] = sA[buf][(am0 + i * 16 + l16) * LDK + kk + lq];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) bfv[j] = sB[cur][(bn0 + j * 16 + l16) * LDK + kk + lq];
+      for (int j = 0; j < TN; ++j) bfv[j] = sB[buf][(bn0 + j * 16 + l16) * LDK + kk + lq];
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            if constexpr (F32)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bfv[j], acc[i][j], 0, 0, 0);
-            else
-              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bfv[j], acc[i][j], 0, 0, 0);
-          }
-      }
-      if (more) store_tiles(cur ^ 1);
-      __syncthreads();
-      cur ^= 1;
+        for (int j = 0; j < TN; ++j) {
+          if constexpr (F32)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bfv[j], acc[i][j], 0, 0, 0);
+          else
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bfv[j], acc[i][j], 0, 0, 0);
+        }
     }
+  };
+  // F32: the running sums are folded into a second set every 512 k, so that a long K range rounds
+  // no more than a short one (relative error of a 136-row sketch of 8192 x 8192 in four ranges of
+  // 2048: 8.1e-7 unfolded, 4.1e-7 folded; eight ranges of 1024 unfolded: 5.7e-7)
+  constexpr int FOLD = 512 / (2 * BK);  // loop passes (of two tiles) between folds
+  constexpr int FM = F32 ? TM : 1, FN = F32 ? TN : 1;
+  ACC sum[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) sum[i][j] = ACC{0, 0, 0, 0};
+  auto fold = [&] {
+    if constexpr (F32) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = ACC{0, 0, 0, 0};
+        }
+    }
+  };
+  // waits for this wave's LDS operations, not for its global loads
+  auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+  // (the pointer alignment of the 16-byte loads: lda, ldb, kbeg and c are even)
+  const int full = kbeg < kend ? (kend - kbeg) / BK : 0;
+  int cur = 0;
+  if (full > 0) {
+    d2 ra0[LA], rb0[LB], ra1[LA], rb1[LB];  // tiles in flight, in turn
+    load_tiles(ra0, rb0, 0);
+    load_tiles(ra1, rb1, min(1, full - 1));
+    store_tiles(ra0, rb0, 0);
+    lds_barrier();
+    // a tile's loads are issued two tiles before its MFMAs
+    for (int t = 0; t < full; t += 2) {
+      load_tiles(ra0, rb0, min(t + 2, full - 1));
+      compute(0);
+      store_tiles(ra1, rb1, 1);
+      lds_barrier();
+      cur = 1;
+      if (t + 1 >= full) break;
+      if (F32 && (t / 2) % FOLD == FOLD - 1) fold();
+      load_tiles(ra1, rb1, min(t + 3, full - 1));
+      compute(1);
+      store_tiles(ra0, rb0, 0);
+      lds_barrier();
+      cur = 0;
+    }
+  }
+  if (kbeg + full * BK < kend) {
+    // (buffer `cur` is free: every wave is past the barrier after its last reads)
+    d2 ra[LA], rb[LB];
+    load_tail(ra, rb, full);
+    store_tiles(ra, rb, cur);
+    lds_barrier();
+    compute(cur);
+  }
+  if constexpr (F32) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] += sum[i][j];
   }
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -619,8 +675,9 @@ static const Cfg kCfgs[] = {{0, 16, 256}, {1, 32, 256}, {2, 48, 256}, {3, 64, 25
                             {5, 16, 256}, {6, 32, 256}, {7, 48, 256}, {8, 64, 256}, {9, 128, 128},
                             {10, 64, 128}, {11, 128, 256}, {12, 128, 128}, {13, 64, 256},
                             {14, 256, 128}, {15, 80, 256}, {16, 96, 256}, {17, 160, 256},
-                            {18, 176, 128}, {19, 208, 128}, {20, 112, 128}, {21, 112, 256}};
-constexpr int kNumCfg = 22;
+                            {18, 176, 128}, {19, 208, 128}, {20, 112, 128}, {21, 112, 256},
+                            {22, 144, 128}, {23, 144, 128}, {24, 112, 128}, {25, 48, 128}};
+constexpr int kNumCfg = 26;
 // ids 5..21: the k-contiguous kernel (gemm_kc_f64_kernel, FP64 or F32 MFMA; 11, 13, 14, 16-21
 // with 512 threads, 12 with 32-wide k-tiles).  15-17 hold a short sketch (ell = 72, 136) in one
 // M-tile, so each k-tile of A is read from L2 once; 18 (11 MFMA rows per wave) covers
@@ -728,6 +785,26 @@ hipError_t launch_cfg(int id, const GemmDev& d, int blocks, hipStream_t st) {
       else if constexpr (PREC == LRA_PREC_F32) hipLaunchKernelGGL((gemm_kc_f64_kernel<112, 256, 1, 8, 16, true>), dim3(blocks), dim3(512), 0, st, d);
       else return hipErrorInvalidValue;
       break;
+    case 22:
+      if constexpr (PREC == LRA_PREC_F64) hipLaunchKernelGGL((gemm_kc_f64_kernel<144, 128, 1, 8, 16, false>), dim3(blocks), dim3(512), 0, st, d);
+      else if constexpr (PREC == LRA_PREC_F32) hipLaunchKernelGGL((gemm_kc_f64_kernel<144, 128, 1, 8, 16, true>), dim3(blocks), dim3(512), 0, st, d);
+      else return hipErrorInvalidValue;
+      break;
+    case 23:
+      if constexpr (PREC == LRA_PREC_F64) hipLaunchKernelGGL((gemm_kc_f64_kernel<144, 128, 1, 8, 32, false>), dim3(blocks), dim3(512), 0, st, d);
+      else if constexpr (PREC == LRA_PREC_F32) hipLaunchKernelGGL((gemm_kc_f64_kernel<144, 128, 1, 8, 32, true>), dim3(blocks), dim3(512), 0, st, d);
+      else return hipErrorInvalidValue;
+      break;
+    case 24:
+      if constexpr (PREC == LRA_PREC_F64) hipLaunchKernelGGL((gemm_kc_f64_kernel<112, 128, 1, 8, 32, false>), dim3(blocks), dim3(512), 0, st, d);
+      else if constexpr (PREC == LRA_PREC_F32) hipLaunchKernelGGL((gemm_kc_f64_kernel<112, 128, 1, 8, 32, true>), dim3(blocks), dim3(512), 0, st, d);
+      else return hipErrorInvalidValue;
+      break;
+    case 25:
+      if constexpr (PREC == LRA_PREC_F64) hipLaunchKernelGGL((gemm_kc_f64_kernel<48, 128, 1, 4, 32, false>), dim3(blocks), dim3(256), 0, st, d);
+      else if constexpr (PREC == LRA_PREC_F32) hipLaunchKernelGGL((gemm_kc_f64_kernel<48, 128, 1, 4, 32, true>), dim3(blocks), dim3(256), 0, st, d);
+      else return hipErrorInvalidValue;
+      break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -783,7 +860,7 @@ int prepare(lra_ctx* ctx, const GemmArgs& g, int cfg, int splits, GemmDev* d, in
   d->A = g.A; d->lda = g.lda; d->transA = g.transA;
   d->B = g.B; d->ldb = g.ldb; d->transB = g.transB;
   d->C = g.C; d->ldc = g.ldc; d->bgather = g.bgather;
-  const int bk = cfg == 12 ? 32 : bk_of(g.prec);
+  const int bk = (cfg == 12 || (cfg >= 23 && cfg <= 25)) ? 32 : bk_of(g.prec);
   i64 kchunk = 0;
   if (g.K <= 0) {
     splits = 1;

@@ -38,6 +38,22 @@ __global__ void gaussian_fill_t_kernel(uint64_t seed, uint64_t stream, i64 rows,
   }
 }
 
+// The same for an even number of rows: normals #2p and #2p + 1 are rows i and i + 1 of one
+// column, so a thread stores both of its pair's (the kernel above evaluates every pair twice:
+// it is bound by the FP64 logarithm and sine-cosine).  520 x 8192: 37 -> 22 us.
+__global__ void gaussian_fill_t2_kernel(uint64_t seed, uint64_t stream, i64 rows, i64 cols,
+                                        double* out, i64 ld) {
+  const i64 h = rows / 2, total = h * cols;
+  for (i64 t = blockIdx.x * (i64)blockDim.x + threadIdx.x; t < total;
+       t += (i64)gridDim.x * blockDim.x) {
+    const i64 j = t % cols, i = t / cols;
+    double z0, z1;
+    lra_normal2(seed, stream, (uint64_t)(j * h + i), &z0, &z1);
+    out[j + 2 * i * ld] = z0;
+    out[j + (2 * i + 1) * ld] = z1;
+  }
+}
+
 __global__ void gaussian_fill_f32_kernel(uint64_t seed, uint64_t stream, i64 rows, i64 cols,
                                          float* out, i64 ld) {
   const i64 total = rows * cols;
@@ -151,8 +167,12 @@ int lra_launch_gaussian_fill(hipStream_t st, uint64_t seed, uint64_t stream_id, 
 int lra_launch_gaussian_fill_t(hipStream_t st, uint64_t seed, uint64_t stream_id, i64 rows,
                                i64 cols, double* out, i64 ld) {
   if (rows <= 0 || cols <= 0) return LRA_OK;
-  hipLaunchKernelGGL(gaussian_fill_t_kernel, dim3(grid_for(rows * cols)), dim3(256), 0, st, seed,
-                     stream_id, rows, cols, out, ld);
+  if (rows % 2 == 0)
+    hipLaunchKernelGGL(gaussian_fill_t2_kernel, dim3(grid_for(rows / 2 * cols)), dim3(256), 0, st,
+                       seed, stream_id, rows, cols, out, ld);
+  else
+    hipLaunchKernelGGL(gaussian_fill_t_kernel, dim3(grid_for(rows * cols)), dim3(256), 0, st, seed,
+                       stream_id, rows, cols, out, ld);
   LRA_LAUNCH_CHECK();
   return LRA_OK;
 }

@@ -294,3 +294,25 @@ def test_dgemm_narrow(gpu, ta, tb, M, N, K, beta):
     gpu.dgemm(A, B, ta, tb, 1.5, C, beta)
     bound = 2.3e-16 * (K + 4) * (1.5 * np.abs(Ah) @ np.abs(Bh) + np.abs(beta * Ch))
     assert (np.abs(host(C) - (1.5 * Ah @ Bh + beta * Ch)) <= bound).all()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("cfg", [5, 8, 10, 12, 14, 17, 18, 19, 21, 22, 23, 24, 25])
+def test_gemm_kc_k_tiles(gpu, monkeypatch, cfg, prec):
+    """The k-contiguous kernel's two tiles in flight: no whole k-tile, one, two, three and many,
+    with and without a remainder (odd K too, the leading dimension even), over one and several
+    K ranges, rows and columns far from filling a tile.  FP64: sums of K terms differ by at most
+    K eps |Omega||A| a term; F32: operands and sums rounded to 24 bits."""
+    import torch
+    eps = 2.3e-16 if prec == "f64" else 1.2e-7
+    for M, N, K, splits in [(3, 5, 7, 1), (17, 130, 16, 1), (40, 300, 32, 1), (130, 70, 33, 1),
+                            (140, 257, 48, 1), (9, 129, 95, 1), (150, 100, 321, 1),
+                            (41, 260, 1031, 2), (200, 140, 700, 3)]:
+        rng = np.random.default_rng(M + N + K)
+        big = torch.from_numpy(rng.standard_normal((N, K + K % 2 + 2))).cuda()
+        A = big[:, :K].t()  # even leading dimension
+        monkeypatch.setenv("LRA_GEMM_CFG", f"{cfg}:{splits}")
+        B = host(gpu.sketch("left", "n", A, M, seed=2, stream=1, precision=prec))
+        Om, Ah = host(gpu.gaussian(M, K, 2, 1)), host(A)
+        bound = (K + 4) * eps * (np.abs(Om) @ np.abs(Ah))
+        assert (np.abs(B - Om @ Ah) <= bound).all(), (M, N, K, splits)
