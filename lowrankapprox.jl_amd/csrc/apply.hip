@@ -63,7 +63,7 @@ extern "C" int lra_dgemm(lra_ctx* c, int transa, int transb, int64_t m, int64_t 
   GemmArgs g;
   g.M = m; g.N = n; g.K = k; g.alpha = alpha; g.beta = beta;
   g.A = A; g.lda = lda; g.transA = transa; g.B = B; g.ldb = ldb; g.transB = transb;
-  g.C = C; g.ldc = ldc; g.bgather = nullptr; g.prec = LRA_PREC_F64;
+  g.C = C; g.ldc = ldc; g.bgather = nullptr; g.prec = LRA_PREC_F64; g.narrow = 1;
   return lra_gemm(c, g);
 }
 
@@ -85,7 +85,7 @@ extern "C" int lra_id_apply(lra_ctx* c, int trans, int64_t k, int64_t n, const i
   const i64 nr = n - k;
   if (nrhs == 0) return LRA_OK;
   GemmArgs g;
-  g.bgather = nullptr; g.prec = LRA_PREC_F64;
+  g.bgather = nullptr; g.prec = LRA_PREC_F64; g.narrow = 1;
   if (trans == 0) {
     if (k == 0) return LRA_OK;
     // Y = X[sk, :], then Y += T X[rd, :]

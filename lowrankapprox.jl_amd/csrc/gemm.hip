@@ -954,7 +954,11 @@ int run_tn_skinny(lra_ctx* ctx, const GemmArgs& g) {
 // 2048: 263 -> 201); with both k-contiguous the tuned tiles read it from LDS as well, and beyond
 // 64 columns narrow is ahead only for short K (7756 x 436 at 128 columns 143 -> 48 us, 200 x
 // 2000 34 -> 16, but 4096 x 4096 105 -> 121).
+// The products inside the factorizations stay on the tiled kernels: a Hermitian factorization's
+// eigenvectors take their signs from the rounding of its core, and the gain there is small
+// (psvdfact of 5689 x 2048 13.5 -> 13.1 ms).
 bool narrow_ok(const GemmArgs& g) {
+  if (!g.narrow) return false;
   if (g.prec != LRA_PREC_F64 || g.bgather != nullptr || g.K < 1 || g.N > 256) return false;
   return g.N <= 64 || g.K <= 2048 || !kc_ok(g);
 }

@@ -294,6 +294,7 @@ struct GemmArgs {
   double* C; i64 ldc;
   const i64* bgather;
   int prec;
+  int narrow = 0;  // a product with few columns may use its own kernel (the factor products)
 };
 int lra_gemm(lra_ctx* ctx, const GemmArgs& g);
 
