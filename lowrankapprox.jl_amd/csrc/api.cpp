@@ -542,7 +542,7 @@ using SketchFn2 = std::function<int(i64, i64, uint64_t, uint64_t, double*)>;
 
 static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opts* o,
                           uint64_t stream_base, SketchFactOut* out, bool pair_ok = true,
-                          const SketchFn2& make2 = nullptr) {
+                          const SketchFn2& make2 = nullptr, bool steady = false) {
   const bool gauss = o->sketch == LRA_SKETCH_RANDN;
   int prec = gauss ? o->precision : LRA_PREC_F64;
   const bool adap = o->sketchfact_adap || o->rank < 0;
@@ -550,6 +550,33 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
   i64* dk = nullptr;
   LRA_CHECK(lra_wsT(c, WS_SCAL, 16, &dk));
   int* dearly = (int*)(dk + 4);
+  // The diagonal of R foreseen from a rejected round of order ell and target t, taken to fall
+  // geometrically from |R(0,0)| to |R(t-1,t-1)|, where |R(i,i)| stands for sigma_i
+  // sqrt(ell - i) (the rows that a Gaussian sketch has left at step i).  A round of order l2 and
+  // target t2 is foreseen to be accepted when its |R(t2-1,t2-1)| is below ptol.  Only
+  // which rounds share a launch depends on it, not what a round gives.  An accepted round that
+  // runs alone saves its partner's sketch and the larger grid (rank 100 of 8192 x 8192: 2.85 ->
+  // 1.72 ms, rank 180 of 2999 x 2999: 3.56 -> 2.63 ms); one that is rejected after all loses
+  // the overlap of the two (about 1.5 ms at orders 264 and 520 of 2999 columns), so the line is
+  // where either outcome is as likely.  steady: the caller's results hang on the sketch's
+  // rounding (a Hermitian factorization's eigenvectors take their signs from it), which a
+  // round's share of a merged product changes; its rounds pair as their sizes allow.
+  double slope = 0.0, depth = 0.0;  // log fall of sigma per step; log(ptol / |R(0,0)|)
+  auto foresee = [&](const i64* hv, i64 ell, i64 t) {
+    double r0 = 0.0, rl = 0.0;
+    std::memcpy(&r0, &hv[2], sizeof(double));
+    std::memcpy(&rl, &hv[3], sizeof(double));
+    const double ptol = std::max(o->atol, o->rtol * r0);
+    slope = depth = 0.0;
+    if (steady || t < 2 || !(rl > 0.0) || !(ptol > 0.0) || !(ptol < r0)) return;
+    slope = (std::log(rl / r0) + 0.5 * std::log((double)ell / (double)(ell - t + 1))) / (double)(t - 1);
+    depth = std::log(ptol / r0);
+  };
+  auto foreseen_accepted = [&](i64 ell, i64 t) {
+    return depth < 0.0 && slope < 0.0 && ell >= t &&
+           slope * (double)(t - 1) + 0.5 * std::log((double)(ell - t + 1) / (double)ell) <
+               depth;
+  };
   for (i64 rnd = 0;;) {
     const i64 ell = samp_of(o, target);
     if (ell <= 0) { lra_set_error("sketch order %lld", (long long)ell); return LRA_E_UNSUPPORTED; }
@@ -562,8 +589,10 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
     // sketch, stop rule and stop_after); the first accepted round is taken, as the
     // sequential loop would.  Round 0 pairs only for wide sketches (N >= 4096): on small
     // problems the pair's larger launch and GEMM cost more than round 0's QR saves, and
-    // small ranks are accepted in round 0.
-    if (pair_ok && adap && prec == LRA_PREC_F64 && (rnd >= 1 || N >= 4096)) {
+    // small ranks are accepted in round 0.  A round that the last rejected one foresees to be
+    // accepted runs alone: its partner would be thrown away (see `foresee`).
+    const bool alone = foreseen_accepted(ell, target);
+    if (pair_ok && adap && prec == LRA_PREC_F64 && (rnd >= 1 || N >= 4096) && !alone) {
       const i64 ell2 = samp_of(o, 2 * target);
       if (ell2 > ell && ell2 < (1 << 20) && N < (1 << 30) &&
           lra_qrcp_pair_fits(c, (int)std::min(ell, N), (int)std::min(ell2, N), (int)N) &&
@@ -602,8 +631,12 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
         }
         const int st = lra_qrcp_pair(c, qs[0], qs[1]);
         if (st == LRA_OK) {
-          i64 hv[2] = {0, 0};
-          LRA_CHECK(read_scalars(c, dk, hv, 2));
+          const bool look = targets[1] <= std::min<i64>(ells[1], N);
+          if (look)
+            LRA_CHECK(lra_launch_two_diagonals(c->stream, qs[1].A, qs[1].lda, targets[1] - 1,
+                                               (double*)(dk + 2)));
+          i64 hv[4] = {0, 0, 0, 0};
+          LRA_CHECK(read_scalars(c, dk, hv, look ? 4 : 2));
           for (int h = 0; h < 2; ++h) {
             if (hv[h] < targets[h]) {
               if (Cp)  // the accepted round's factored rows, compact (ld = its order)
@@ -615,6 +648,7 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
               return LRA_OK;
             }
           }
+          if (look) foresee(hv, ells[1], targets[1]);
           target *= 4;
           rnd += 2;
           continue;
@@ -648,13 +682,10 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
     q.k_out = dk; q.early_out = dearly;
     LRA_CHECK(lra_qrcp(c, q));
     // with rtol below the floor, a rejected low-precision round also reports |R(0,0)| (the
-    // largest column norm) and |R(t-1,t-1)|, t = target: R is written back on every exit
-    const bool look = adap && lowp && o->rtol < floor && target >= 1 && target <= l;
-    if (look) {
-      LRA_HIP(hipMemcpyAsync(dk + 2, B, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      LRA_HIP(hipMemcpyAsync(dk + 3, B + (target - 1) * (ell + 1), sizeof(double),
-                             hipMemcpyDeviceToDevice, c->stream));
-    }
+    // largest column norm) and |R(t-1,t-1)|, t = target: R is written back on every exit; so does
+    // an FP64 round whose successor may pair
+    const bool look = adap && target >= 1 && target <= l && (lowp ? o->rtol < floor : pair_ok);
+    if (look) LRA_CHECK(lra_launch_two_diagonals(c->stream, B, ell, target - 1, (double*)(dk + 2)));
     i64 hv[4] = {0, 0, 0, 0};
     LRA_CHECK(read_scalars(c, dk, hv, look ? 4 : 1));
     const i64 hk = hv[0];
@@ -664,7 +695,8 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
       prec = LRA_PREC_F64;
       continue;
     }
-    if (!accept && look) {
+    if (!accept && look && !lowp) foresee(hv, ell, target);
+    if (!accept && look && lowp) {
       // the next round (twice the target) is run in FP64 from the start when this round's
       // last pivot is already within kFloorAhead of the floor: a low-precision attempt would
       // most likely stop on the floor and be recomputed.  Only the precision of a round
@@ -787,7 +819,7 @@ static int op_sketch(lra_ctx* c, int trans, const LraSrc& s, i64 ell, uint64_t s
 // sketchfact(:left, trans, A) on a dense matrix (any sketch) or an operator (Gaussian only,
 // the caller has applied lra_opts_for_operator), with sketch_randn_niter power iterations.
 static int sketchfact_left(lra_ctx* c, int trans, const LraSrc& s, const lra_opts* o,
-                           SketchFactOut* out, uint64_t stream_base = 0) {
+                           SketchFactOut* out, uint64_t stream_base = 0, bool steady = false) {
   const i64 N = trans == LRA_TRANS_N ? s.n : s.m;  // columns of op(A)
   const i64 niter = o->sketch == LRA_SKETCH_RANDN ? o->sketch_randn_niter : 0;
   bool herm = false;
@@ -816,7 +848,7 @@ static int sketchfact_left(lra_ctx* c, int trans, const LraSrc& s, const lra_opt
       return sketch_gaussian_left2(c, trans, s.m, s.n, s.A, s.lda, ell0, ell1, o->seed, s0, s1,
                                    C);
     };
-  return sketchfact_run(c, N, make, o, stream_base, out, !s.op(), make2);
+  return sketchfact_run(c, N, make, o, stream_base, out, !s.op(), make2, steady);
 }
 
 int lra_src_getcols(lra_ctx* c, const LraSrc& s, int trans, const i64* idx, i64 k, double* C,
@@ -894,7 +926,7 @@ static int finish_id(lra_ctx* c, const SketchFactOut& f, i64 N, const lra_opts* 
                      lra_id_out* out, const RefineFn& refine);
 
 int lra_idfact_src(lra_ctx* c, int trans, const LraSrc& s, const lra_opts* opts,
-                   lra_id_out* out) {
+                   lra_id_out* out, bool steady) {
   if (chkopts(opts) != LRA_OK) return -7;
   lra_opts o = *opts;
   o.pqrfact_retval = LRA_RET_T;
@@ -919,7 +951,7 @@ int lra_idfact_src(lra_ctx* c, int trans, const LraSrc& s, const lra_opts* opts,
     f.B = B; f.Bsave = nullptr; f.ell = P; f.N = N; f.jpvt = jpvt; f.tau = tau; f.k = k;
     f.rounds = 1; f.prec = LRA_PREC_F64; f.stream_id = 0;
   } else {
-    LRA_CHECK(sketchfact_left(c, trans, s, &o, &f));
+    LRA_CHECK(sketchfact_left(c, trans, s, &o, &f, 0, steady));
   }
   return finish_id(c, f, N, &o, out, [&](const i64* sk, const i64* rd, double* T, i64 ldt) {
     if (s.op()) return (int)LRA_OK;  // operators are sketched in FP64 (no refinement)

@@ -154,7 +154,8 @@ struct IdOut {
   i64 rounds;
 };
 
-int run_id(lra_ctx* c, int trans, const LraSrc& src, const lra_opts* o, IdOut* r) {
+int run_id(lra_ctx* c, int trans, const LraSrc& src, const lra_opts* o, IdOut* r,
+           bool steady = false) {
   const i64 m = src.m, n = src.n;
   const i64 N = trans == LRA_TRANS_N ? n : m;
   r->N = N;
@@ -165,7 +166,7 @@ int run_id(lra_ctx* c, int trans, const LraSrc& src, const lra_opts* o, IdOut* r
   LRA_CHECK(lra_wsT(c, WS_F2, (size_t)std::max<i64>(N, 1), &p));
   lra_id_out out{};
   out.sk = sk; out.rd = rd; out.T = nullptr; out.ldt = 0;
-  LRA_CHECK(lra_idfact_src(c, trans, src, o, &out));
+  LRA_CHECK(lra_idfact_src(c, trans, src, o, &out, steady));
   r->k = out.k;
   r->sk = sk; r->rd = rd; r->p = p;
   r->T = out.T; r->ldt = out.ldt; r->rounds = out.rounds;
@@ -498,7 +499,7 @@ static int pheig_impl(lra_ctx* c, const LraSrc& src, const lra_opts* opts, bool 
   const lra_opts o = *opts;
   const i64 n = src.n;
   IdOut id;
-  LRA_CHECK(run_id(c, LRA_TRANS_N, src, &o, &id));
+  LRA_CHECK(run_id(c, LRA_TRANS_N, src, &o, &id, /*steady=*/true));
   const i64 k = id.k, N = n;
   out->k = out->kn = out->kp = 0;
   if (k == 0) return LRA_OK;

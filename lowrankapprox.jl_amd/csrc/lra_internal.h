@@ -106,8 +106,9 @@ int lra_src_getcols(lra_ctx* c, const LraSrc& s, int trans, const i64* idx, i64 
 // D (k x k) = A[idx, idx] (getindex(L, rows, cols), src/linop.jl:70-74)
 int lra_src_principal(lra_ctx* c, const LraSrc& s, const i64* idx, i64 k, double* D, i64 ldd);
 // idfact(trans, A, opts) on either kind of source (src/id.jl:434-447)
+// (steady: rounds pair by their size alone)
 int lra_idfact_src(lra_ctx* c, int trans, const LraSrc& s, const lra_opts* opts,
-                   lra_id_out* out);
+                   lra_id_out* out, bool steady = false);
 // the reference's chkopts!(opts, A) for an operator (src/LowRankApprox.jl:142-148): a sketch
 // other than randn is replaced by randn with a warning (verb != 0)
 void lra_opts_for_operator(lra_opts* o);
@@ -350,6 +351,7 @@ int lra_launch_transpose(hipStream_t st, i64 m, i64 n, const double* A, i64 lda,
                          i64 ldo);
 int lra_launch_copy2d(hipStream_t st, i64 m, i64 n, const double* A, i64 lda, double* out,
                       i64 ldo);
+int lra_launch_two_diagonals(hipStream_t st, const double* A, i64 lda, i64 i, double* out);
 int lra_launch_split_ids(hipStream_t st, i64 n, i64 k, const i64* jpvt, i64* sk, i64* rd);
 // S (rows x k) = one-hot columns e_idx[j] (idx 1-based)
 int lra_launch_onehot(hipStream_t st, i64 rows, i64 k, const i64* idx, double* S, i64 lds);

@@ -74,6 +74,11 @@ __global__ void gather_rows_kernel(i64 k, i64 n, const double* A, i64 lda, const
     out[i + j * ldo] = A[(rows[i] - 1) + j * lda];
 }
 
+// out[0] = |A(0, 0)|, out[1] = |A(i, i)|
+__global__ void two_diagonals_kernel(const double* A, i64 lda, i64 i, double* out) {
+  out[threadIdx.x] = fabs(A[threadIdx.x == 0 ? 0 : i * (lda + 1)]);
+}
+
 __global__ void split_ids_kernel(i64 n, i64 k, const i64* jpvt, i64* sk, i64* rd) {
   for (i64 i = blockIdx.x * (i64)blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
     if (i < k) { if (sk) sk[i] = jpvt[i]; }
@@ -156,6 +161,12 @@ int lra_launch_gather_rows(hipStream_t st, i64 k, i64 n, const double* A, i64 ld
   if (n > 65535) { lra_set_error("gather_rows: n too large"); return LRA_E_UNSUPPORTED; }
   dim3 grid((unsigned)std::min<i64>((k + 255) / 256, 64), (unsigned)n);
   hipLaunchKernelGGL(gather_rows_kernel, grid, dim3(256), 0, st, k, n, A, lda, rows, out, ldo);
+  LRA_LAUNCH_CHECK();
+  return LRA_OK;
+}
+
+int lra_launch_two_diagonals(hipStream_t st, const double* A, i64 lda, i64 i, double* out) {
+  hipLaunchKernelGGL(two_diagonals_kernel, dim3(1), dim3(2), 0, st, A, lda, i, out);
   LRA_LAUNCH_CHECK();
   return LRA_OK;
 }
