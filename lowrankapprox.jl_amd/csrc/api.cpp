@@ -680,6 +680,12 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
     q.jpvt = jpvt; q.tau = tau; q.vn1 = nullptr;
     q.vn2 = nullptr; q.stop_after = adap ? (int)std::min<i64>(target, 1 << 30) : 0;
     q.k_out = dk; q.early_out = dearly;
+    // Large sketches whose diagonal is foreseen to fall slowly go to the HBM kernels' blocks of
+    // steps, whose length is about the fall of the norms among the largest columns.  A step by
+    // the register-resident grid and in blocks, at a fall of 1, 2, 3, 4.5% a step: 520 x 8192
+    // 8.9 us and 7.6, 8.5, 9.2, 10.2; 520 x 3758 7.3 and 6.2, 6.7, 7.3, 7.9; 1032 x 3758 9.3-9.9
+    // and 6.6, 7.4, 8.5, 9.9.
+    q.blocks = !lowp && slope < 0.0 && ((ell >= 500 && slope > -0.02) || (ell >= 900 && slope > -0.035));
     LRA_CHECK(lra_qrcp(c, q));
     // with rtol below the floor, a rejected low-precision round also reports |R(0,0)| (the
     // largest column norm) and |R(t-1,t-1)|, t = target: R is written back on every exit; so does

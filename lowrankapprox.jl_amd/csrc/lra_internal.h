@@ -319,6 +319,7 @@ struct QrcpCall {
   int* early_out;            // device scalar: 1 when stop_after fired
   int exact_tail;            // the columns past the rank are read by the caller: no step is
                              // applied beyond the one that ends the factorization
+  int blocks;                // the norms are foreseen to fall slowly: blocks of steps in HBM
 };
 int lra_qrcp(lra_ctx* ctx, const QrcpCall& q);
 // Two mode-0 factorizations of equal n (q0.m <= q1.m) in one co-resident launch;
@@ -329,6 +330,8 @@ int lra_qrcp_pair(lra_ctx* ctx, const QrcpCall& q0, const QrcpCall& q1);
 // qrcp_global.hip: the same (mode 0) with the sketch in HBM, for sketches beyond the
 // register-resident kernel
 int lra_qrcp_global(lra_ctx* ctx, const QrcpCall& q);
+// whether an m x n sketch can run there in blocks of steps (workspace and exchange area)
+bool lra_qrcp_blocks_fit(lra_ctx* ctx, int m, int n);
 
 // trsm.hip: T = R11 \ R12; in-place op(U) X = B with U the upper k x k triangle of R
 int lra_launch_id_T(hipStream_t st, i64 k, i64 n, const double* R, i64 ldr, double* T, i64 ldt);

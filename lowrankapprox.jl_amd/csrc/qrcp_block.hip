@@ -21,7 +21,7 @@
 // between, so the dlaqps block ends fall on the same steps as step by step.
 //
 // Measured on a 2056 x 3758 sketch of sigma_i = exp(-0.01 (i-1)), 1152 steps in 128 blocks:
-// 11.0 ms against 26.9 ms of single steps.  A block at s = 500 takes 86 us: select 11 and gram 11
+// 10.2 ms against 26.9 ms of single steps.  A block at s = 500 takes 80 us: select 6 and gram 11
 // (latency: dependent loads of one workgroup, and 2300 rows over 16 waves), panel 32 (the chain
 // of pivots, 0.7 us each, and of columns, 1.6 us each), apply 32 (reading and writing the
 // trailing matrix at about 5 TB/s).  128 candidates because their Gram matrix fits LDS, where a
@@ -44,83 +44,96 @@ constexpr int QT = 1024;  // threads of every kernel here
 
 // ---- bookkeeping and candidates ---------------------------------------------------------
 
+// VPT positions per thread in registers (n <= 1024 VPT), else read three times (VPT = 0).
+// Bound by its chain of dependent loads and barriers: the norms load while thread 0 does the
+// bookkeeping, each wave reduces the waves' maxima itself, and only norms of at least half the
+// largest enter the histogram (256 bins, one wave's scan).
+template <int VPT>
 __global__ __launch_bounds__(QT) void qb_select(int n, int kmax, int nb, int stop_after,
                                                 const double* __restrict__ vn1,
                                                 const double* __restrict__ diag, int* at,
                                                 int* cand, FState* st) {
-  constexpr int VPT = 16, NBIN = 1024;
-  __shared__ int s_done, s_s, s_cnt, s_T, s_ap;
-  __shared__ double s_mx[QT / 64], s_tau[QT / 64];
-  __shared__ int s_mp[QT / 64], s_ws[QT / 64];
+  constexpr int NW = QT / 64, NBIN = 256;
+  __shared__ int s_done, s_cnt, s_T;
+  __shared__ double s_mx[NW], s_tau[NW];
+  __shared__ int s_mp[NW];
   __shared__ int hist[NBIN];
   if (st->done) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  hist[tid] = 0;
+  const int s0 = st->s, b = st->b, s = s0 + b;  // (unless the block holds the last step)
+  auto norm_at = [&](int p) {
+    const double x = vn1[at[p]];
+    return x >= 0.0 ? x : -1.0;  // (a NaN norm takes no part)
+  };
+  double v[VPT ? VPT : 1];
+  int c[VPT ? VPT : 1];
+  if constexpr (VPT > 0) {
+#pragma unroll
+    for (int r = 0; r < VPT; ++r) {
+      const int p = s + tid + r * QT;
+      c[r] = p < n ? at[p] : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < VPT; ++r) {
+      const double x = c[r] >= 0 ? vn1[c[r]] : -1.0;
+      v[r] = x >= 0.0 ? x : -1.0;
+    }
+  }
+  if (tid < NBIN) hist[tid] = 0;
   if (tid == 0) {
-    const int s = st->s, b = st->b;
     const unsigned mask = st->mask;
     int done = 0, e = b;
-    for (int t = 0; t < b && !done; ++t) {
-      const int step = s + t, s1 = step + 1;
-      if (!((step - st->j0 + 1 == st->jb) || ((mask >> t) & 1) || s1 == kmax)) continue;
-      const double ptol = st->ptol;
-      bool stop = false;
-      if (fabs(diag[step]) <= ptol) {
-        int i = st->j0;
-        for (; i < step; ++i)
-          if (fabs(diag[i]) <= ptol) break;
-        st->k = i;
-        stop = true;
+    if (b > 0) {
+      int j0 = st->j0, jb = st->jb;
+      for (int t = 0; t < b && !done; ++t) {
+        const int step = s0 + t, s1 = step + 1;
+        if (!((step - j0 + 1 == jb) || ((mask >> t) & 1) || s1 == kmax)) continue;
+        const double ptol = st->ptol;
+        bool stop = false;
+        if (fabs(diag[step]) <= ptol) {
+          int i = j0;
+          for (; i < step; ++i)
+            if (fabs(diag[i]) <= ptol) break;
+          st->k = i;
+          stop = true;
+        }
+        if (!stop && s1 == kmax) { st->k = kmax; stop = true; }
+        if (!stop && stop_after > 0 && s1 >= stop_after) {
+          st->k = s1;
+          st->early = 1;
+          stop = true;
+        }
+        if (stop) {
+          done = 1;
+          e = t + 1;
+        } else {
+          j0 = s1;
+          jb = min(nb, kmax - s1);
+        }
       }
-      if (!stop && s1 == kmax) { st->k = kmax; stop = true; }
-      if (!stop && stop_after > 0 && s1 >= stop_after) {
-        st->k = s1;
-        st->early = 1;
-        stop = true;
-      }
-      if (stop) {
-        done = 1;
-        e = t + 1;
-      } else {
-        st->j0 = s1;
-        st->jb = min(nb, kmax - s1);
+      st->j0 = j0;
+      st->jb = jb;
+      // the swaps of steps after the one that stopped are taken back, last first
+      const int* swp = cand + 2 * QB_C;
+      for (int t = b - 1; t >= e; --t) {
+        const int p = swp[t], cc = at[s0 + t];
+        at[s0 + t] = at[p];
+        at[p] = cc;
       }
     }
-    // the swaps of steps after the one that stopped are taken back, last first
-    const int* swp = cand + 2 * QB_C;
-    for (int t = b - 1; t >= e; --t) {
-      const int p = swp[t], c = at[s + t];
-      at[s + t] = at[p];
-      at[p] = c;
-    }
-    st->s = s + e;
+    st->s = s0 + e;
     st->b = 0;
     st->mask = 0;
     st->sprev = -1;
     st->done = done;
     s_done = done;
-    s_s = s + e;
     s_cnt = 0;
     s_T = NBIN;
   }
-  __syncthreads();
-  if (s_done) return;
-  const int s = s_s, tr = n - s;
-  // trailing norms (a NaN norm takes no part)
-  double v[VPT];
-  const bool held = tr <= QT * VPT;
-  auto norm_at = [&](int p) {
-    const double x = vn1[at[p]];
-    return x >= 0.0 ? x : -1.0;
-  };
+  // the largest norm, lowest position first among equals
   double bv = -1.0;
   int bp = INT_MAX;
-  if (held) {
-#pragma unroll
-    for (int r = 0; r < VPT; ++r) {
-      const int p = s + tid + r * QT;
-      v[r] = p < n ? norm_at(p) : -1.0;
-    }
+  if constexpr (VPT > 0) {
 #pragma unroll
     for (int r = 0; r < VPT; ++r)
       if (v[r] > bv) { bv = v[r]; bp = s + tid + r * QT; }
@@ -138,83 +151,93 @@ __global__ __launch_bounds__(QT) void qb_select(int n, int kmax, int nb, int sto
     s_mp[wave] = wl < 0 ? INT_MAX : wp;
   }
   __syncthreads();
-  if (tid == 0) {
-    double cv = s_mx[0];
-    int cp = s_mp[0];
-    for (int w = 1; w < QT / 64; ++w)
-      if (s_mx[w] > cv || (s_mx[w] == cv && s_mp[w] < cp)) { cv = s_mx[w]; cp = s_mp[w]; }
-    s_mx[0] = cv;
-    s_ap = cp;
-    if (cp < s || cp >= n) {  // no candidate (NaN norms)
+  if (s_done) return;
+  const double lv = lane < NW ? s_mx[lane] : -1.0;
+  const int lp = lane < NW ? s_mp[lane] : INT_MAX;
+  double vmax;
+  const int ml = wave_argmax(lv, lp, 1, &vmax);
+  if (ml < 0) {  // no candidate (NaN norms)
+    if (tid == 0) {
       st->k = s;
       st->done = 1;
-      s_done = 1;
-    } else {
-      cand[0] = at[cp];
-      cand[QB_C] = cp;
     }
+    return;
   }
-  __syncthreads();
-  if (s_done) return;
-  const double vmax = s_mx[0];
-  const int ap = s_ap;
+  const int ap = __builtin_amdgcn_readlane(lp, ml);
+  if (tid == 0) {
+    cand[0] = at[ap];
+    cand[QB_C] = ap;
+  }
   // squares of norms outside this range do not fit the Gram matrix: single steps
   if (!(vmax >= 1e-140 && vmax <= 1e140)) {
     if (tid == 0) st->ncand = 0;
     return;
   }
-  const double sc = (double)NBIN / vmax;
-  auto bin_of = [&](double x) { return min(NBIN - 1, (int)(x * sc)); };
-  if (held) {
+  // bin of a norm: 256 bins from half the largest to the largest, -1 below
+  const double sc = 2.0 * NBIN / vmax;
+  auto bin_of = [&](double x) { return x * 2.0 >= vmax ? min(NBIN - 1, (int)(x * sc) - NBIN) : -1; };
+  auto count = [&](double x) {
+    const int k = bin_of(x);
+    if (k >= 0) atomicAdd(&hist[k], 1);
+  };
+  if constexpr (VPT > 0) {
 #pragma unroll
-    for (int r = 0; r < VPT; ++r)
-      if (v[r] >= 0.0) atomicAdd(&hist[bin_of(v[r])], 1);
+    for (int r = 0; r < VPT; ++r) count(v[r]);
   } else {
-    for (int p = s + tid; p < n; p += QT) {
-      const double x = norm_at(p);
-      if (x >= 0.0) atomicAdd(&hist[bin_of(x)], 1);
-    }
+    for (int p = s + tid; p < n; p += QT) count(norm_at(p));
   }
   __syncthreads();
   // the lowest bin T with at most QB_C - 1 columns in the bins from T up
-  int c = hist[tid];
-  for (int d = 1; d < 64; d <<= 1) {
-    const int o = __shfl_down(c, d, 64);
-    if (lane + d < 64) c += o;
+  if (wave == 0) {
+    int h[4], tot = 0;
+#pragma unroll
+    for (int k = 3; k >= 0; --k) {
+      h[k] = hist[4 * lane + k];
+      tot += h[k];
+    }
+    int up = tot;  // columns in this lane's bins and all above
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_down(up, d, 64);
+      if (lane + d < 64) up += o;
+    }
+    up -= tot;
+    if (up < QB_C) {
+#pragma unroll
+      for (int k = 3; k >= 0; --k) {
+        if (up < QB_C && up + h[k] >= QB_C) s_T = 4 * lane + k + 1;  // (one lane at the most)
+        up += h[k];
+      }
+      if (lane == 0 && up < QB_C) s_T = 0;
+    }
   }
-  if (lane == 0) s_ws[wave] = c;
-  __syncthreads();
-  for (int w = wave + 1; w < QT / 64; ++w) c += s_ws[w];
-  const int up = c - hist[tid];  // columns in the bins above this one
-  if (c >= QB_C && up < QB_C) s_T = tid + 1;
-  if (tid == 0 && c < QB_C) s_T = 0;
   __syncthreads();
   const int T = s_T;
   double tau = -1.0;
-  auto place = [&](double x, int p) {
+  auto place = [&](double x, int p, int col) {
     if (p == ap || x < 0.0) return;
     if (bin_of(x) >= T) {
       const int i = 1 + atomicAdd(&s_cnt, 1);
-      cand[i] = at[p];
+      cand[i] = col;
       cand[QB_C + i] = p;
     } else {
       tau = fmax(tau, x);
     }
   };
-  if (held) {
+  if constexpr (VPT > 0) {
 #pragma unroll
-    for (int r = 0; r < VPT; ++r) place(v[r], s + tid + r * QT);
+    for (int r = 0; r < VPT; ++r) place(v[r], s + tid + r * QT, c[r]);
   } else {
-    for (int p = s + tid; p < n; p += QT) place(norm_at(p), p);
+    for (int p = s + tid; p < n; p += QT) place(norm_at(p), p, at[p]);
   }
   tau = wave_max(tau);
   if (lane == 0) s_tau[wave] = tau;
   __syncthreads();
-  if (tid == 0) {
-    double t2 = s_tau[0];
-    for (int w = 1; w < QT / 64; ++w) t2 = fmax(t2, s_tau[w]);
-    st->tau = t2;
-    st->ncand = min(QB_C, 1 + s_cnt);
+  if (wave == 0) {
+    tau = wave_max(lane < NW ? s_tau[lane] : -1.0);
+    if (lane == 0) {
+      st->tau = tau;
+      st->ncand = min(QB_C, 1 + s_cnt);
+    }
   }
 }
 
@@ -717,8 +740,13 @@ __global__ __launch_bounds__(QT) void qb_apply(int m, int n, int lastrk, double*
 
 void launch_select(lra_ctx* c, const QrcpCall& q, const QbWork& w, const int* at, double* vn1,
                    const double* diag, FState* st) {
-  hipLaunchKernelGGL(qb_select, dim3(1), dim3(QT), 0, c->stream, q.n, q.kmax, q.nb, q.stop_after,
-                     vn1, diag, const_cast<int*>(at), w.cand, st);
+#define QS_ARGS dim3(1), dim3(QT), 0, c->stream, q.n, q.kmax, q.nb, q.stop_after, vn1, diag, \
+                const_cast<int*>(at), w.cand, st
+  if (q.n <= 4 * QT) hipLaunchKernelGGL(qb_select<4>, QS_ARGS);
+  else if (q.n <= 8 * QT) hipLaunchKernelGGL(qb_select<8>, QS_ARGS);
+  else if (q.n <= 16 * QT) hipLaunchKernelGGL(qb_select<16>, QS_ARGS);
+  else hipLaunchKernelGGL(qb_select<0>, QS_ARGS);
+#undef QS_ARGS
 }
 
 template <int RP, int NB>

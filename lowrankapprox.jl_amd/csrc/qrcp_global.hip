@@ -1395,6 +1395,17 @@ void launch_fused(hipStream_t s0, int s, int s_first, const QrcpCall& q, int las
 
 }  // namespace
 
+bool lra_qrcp_blocks_fit(lra_ctx* c, int m, int n) {
+  const char *fe = getenv("LRA_QG_FUSED"), *be = getenv("LRA_QG_BLOCK");
+  if ((fe && fe[0] == '0') || (be && be[0] == '0') || m > 8192 || n >= (int)F_NONE) return false;
+  double* w = nullptr;
+  void* area = nullptr;
+  bool uc = false;
+  return lra_wsT(c, WS_QGT, (size_t)m * n, &w) == LRA_OK &&
+         lra_wsT(c, WS_QGB, lra_qb_doubles(m), &w) == LRA_OK &&
+         lra_coop_area(c, kPartOff + 16 * (size_t)n, &area, &uc) == LRA_OK && uc;
+}
+
 // geqp3_adap (mode 0 of QrcpCall) on a sketch of any size, in HBM.
 int lra_qrcp_global(lra_ctx* c, const QrcpCall& q) {
   if (q.mode != 0) {
@@ -1462,7 +1473,7 @@ int lra_qrcp_global(lra_ctx* c, const QrcpCall& q) {
         return LRA_OK;
       };
       // Blocks of steps where their workspace fits the budget (LRA_QG_BLOCK=0: single steps
-      // only).  A block takes 57 to 92 us (rows 900 to 2056, 3758 columns) against 10 to 24 us
+      // only).  A block takes 50 to 88 us (rows 900 to 2056, 3758 columns) against 10 to 24 us
       // for a single step, about four of them, so where the blocks come out shorter than
       // kShort steps on average (many columns of nearly equal norm, or norms outside the
       // blocks' range) single steps run, twice as many each time.
