@@ -473,6 +473,68 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
     }
 }
 
+// C (M x N) = alpha op(A) op(B) + beta C, FP64, for K <= 64 and a tall C (the blocked QR's
+// X -= V W): 16 rows by 64 columns a wave, every operand of 32 k loaded at once and straight into
+// the MFMA registers, no LDS.  The product is formed transposed, D = op(B)' op(A)', so that 16
+// lanes hold 16 consecutive rows of a column of C.  Bound by reading and writing C: 5689 x 199
+// at K = 32 takes 9 us; the tiled kernel, 90 workgroups of 128 x 128, took 58.  The k of an MFMA
+// are 4 j + 0..3 in turn, the tiled kernel's order, so both give the same bits.
+__global__ __launch_bounds__(256) void gemm_short_k_kernel(int M, int N, int K,
+                                                           const double* __restrict__ A, i64 am,
+                                                           i64 ak, const double* __restrict__ B,
+                                                           i64 bk, i64 bn, double alpha, double beta,
+                                                           double* __restrict__ C, i64 ldc) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, q = lane >> 4;
+  const int m = (int)blockIdx.x * 64 + wave * 16 + l16, n0 = (int)blockIdx.y * 64;
+  const double* pa = A + (i64)min(m, M - 1) * am;
+  const double* pb[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) pb[j] = B + (i64)min(n0 + 16 * j + l16, N - 1) * bn;
+  // register r of tile j is column n0 + 16 j + q + 4 r
+  double c[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = n0 + 16 * j + q + 4 * r;
+      const bool ok = beta != 0.0 && m < M && n < N;
+      const double x = C[ok ? m + (i64)n * ldc : 0];
+      c[j][r] = ok ? x : 0.0;
+    }
+  d4 acc[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc[j] = d4{0, 0, 0, 0};
+  for (int k0 = 0; k0 < K; k0 += 32) {
+    double a[8], b[4][8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int k = k0 + 4 * u + q;
+      const i64 kc = min(k, K - 1);  // (loaded in range, zero from K on)
+      const double xa = pa[kc * ak];
+      a[u] = k < K ? xa : 0.0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const double xb = pb[j][kc * bk];
+        b[j][u] = k < K ? xb : 0.0;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][u], a[u], acc[j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = n0 + 16 * j + q + 4 * r;
+      if (m < M && n < N)
+        C[m + (i64)n * ldc] = beta != 0.0 ? alpha * acc[j][r] + beta * c[j][r] : alpha * acc[j][r];
+    }
+}
+
 // C (M x N <= 16 NT) = alpha op(A) op(B) + beta C, FP64, one 32-row tile and one K range per
 // workgroup; each wave takes every fourth 16-deep step of the range and the four partial tiles
 // meet in LDS.  Operands go from memory to the MFMA registers: with k = 4 q + r for register r of
@@ -1030,15 +1092,28 @@ TuneVal heuristic(const GemmArgs& g, int num_cu) {
   return {cfg, s};
 }
 
-// A short-K product with a tall C (the blocked QR's X -= V W and its like) as the transposed
-// product C' = op(B)' op(A)' stored transposed: the MFMA output tile then puts 16 consecutive
-// rows of one column of C in 16 consecutive lanes, so the read-modify-write of C is
-// coalesced.  One K-range, the general kernel's configuration for the swapped shape.
+// A short-K product with a tall C (the blocked QR's X -= V W and its like): in FP64 on
+// gemm_short_k_kernel.  The low precisions form the transposed product C' = op(B)' op(A)' stored
+// transposed: the MFMA output tile then puts 16 consecutive rows of one column of C in 16
+// consecutive lanes, so the read-modify-write of C is coalesced.  One K-range, the general
+// kernel's configuration for the swapped shape.
 bool ct_ok(const GemmArgs& g) {
   return g.bgather == nullptr && g.K <= 64 && g.M >= 256 && g.M >= 2 * g.N;
 }
 
 int run_ct(lra_ctx* ctx, const GemmArgs& g) {
+  if (g.prec == LRA_PREC_F64 && g.K >= 1) {
+    const dim3 grid((unsigned)((g.M + 63) / 64), (unsigned)((g.N + 63) / 64));
+    hipLaunchKernelGGL(gemm_short_k_kernel, grid, dim3(256), 0, ctx->stream, (int)g.M, (int)g.N,
+                       (int)g.K, g.A, g.transA ? g.lda : 1, g.transA ? 1 : g.lda, g.B,
+                       g.transB ? g.ldb : 1, g.transB ? 1 : g.ldb, g.alpha, g.beta, g.C, g.ldc);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      lra_set_error("short-K gemm launch: %s", hipGetErrorString(e));
+      return LRA_E_HIP;
+    }
+    return LRA_OK;
+  }
   GemmArgs s = g;
   s.M = g.N; s.N = g.M;
   s.A = g.B; s.lda = g.ldb; s.transA = !g.transB;
