@@ -473,13 +473,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
     }
 }
 
-// C (M x N) = alpha op(A) op(B) + beta C, FP64, for K <= 64 and a tall C (the blocked QR's
-// X -= V W): 16 rows by 64 columns a wave, every operand of 32 k loaded at once and straight into
-// the MFMA registers, no LDS.  The product is formed transposed, D = op(B)' op(A)', so that 16
-// lanes hold 16 consecutive rows of a column of C.  Bound by reading and writing C: 5689 x 199
-// at K = 32 takes 9 us; the tiled kernel, 90 workgroups of 128 x 128, took 58.  The k of an MFMA
-// are 4 j + 0..3 in turn, the tiled kernel's order, so both give the same bits.
-__global__ __launch_bounds__(256) void gemm_short_k_kernel(int M, int N, int K,
+// C (M x N) = alpha op(A) op(B) + beta C, FP64, any storage order, for products whose 128 x 128
+// tiles would be few (the blocked QR's X -= V W, a factor's Q times its small core): 16 rows by 64
+// columns a wave, operands straight into the MFMA registers 16 k ahead, no LDS.  The product is
+// formed transposed, D = op(B)' op(A)', so that 16 lanes hold 16 consecutive rows of a column of
+// C.  Bound by reading and writing C for a short K (5689 x 199 at K = 32: 10 us, tiled 58: 90
+// workgroups), by L1 reads of op(B) for a long one (5689 x 300 at K = 231: 50 us, tiled 132).  The
+// k of an MFMA are 4 j + 0..3 in turn, the tiled kernel's order, so both give the same bits.
+__global__ __launch_bounds__(256) void gemm_direct_kernel(int M, int N, int K,
                                                            const double* __restrict__ A, i64 am,
                                                            i64 ak, const double* __restrict__ B,
                                                            i64 bk, i64 bn, double alpha, double beta,
@@ -505,10 +506,10 @@ __global__ __launch_bounds__(256) void gemm_short_k_kernel(int M, int N, int K,
   d4 acc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = d4{0, 0, 0, 0};
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    double a[8], b[4][8];
+  double a[4], b[4][4];  // the next 16 k
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < 4; ++u) {
       const int k = k0 + 4 * u + q;
       const i64 kc = min(k, K - 1);  // (loaded in range, zero from K on)
       const double xa = pa[kc * ak];
@@ -519,11 +520,22 @@ __global__ __launch_bounds__(256) void gemm_short_k_kernel(int M, int N, int K,
         b[j][u] = k < K ? xb : 0.0;
       }
     }
+  };
+  load(0);
+  for (int k0 = 0; k0 < K; k0 += 16) {
+    double ca[4], cb[4][4];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < 4; ++u) {
+      ca[u] = a[u];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cb[j][u] = b[j][u];
+    }
+    if (k0 + 16 < K) load(k0 + 16);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][u], a[u], acc[j], 0, 0, 0);
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(cb[j][u], ca[u], acc[j], 0, 0, 0);
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -1092,8 +1104,30 @@ TuneVal heuristic(const GemmArgs& g, int num_cu) {
   return {cfg, s};
 }
 
+// Where gemm_direct_kernel takes a product of operands that are not both k-contiguous: up to 512 k
+// (one K range in either form) and 2 M elements of C.  Tiled -> direct: 1817 x 300 at K = 231 66
+// -> 29 us, 1000 x 1000 at K = 500 89 -> 61, 5689 x 300 (1.7 M) at K = 500 250 -> 103; 4000 x
+// 1000 (4 M) at K = 231 75 -> 91.
+bool direct_ok(const GemmArgs& g) {
+  return g.prec == LRA_PREC_F64 && g.bgather == nullptr && g.K >= 1 && g.K <= 512 &&
+         g.M * g.N <= (1ll << 21) && !kc_ok(g);
+}
+
+int run_direct(lra_ctx* ctx, const GemmArgs& g) {
+  const dim3 grid((unsigned)((g.M + 63) / 64), (unsigned)((g.N + 63) / 64));
+  hipLaunchKernelGGL(gemm_direct_kernel, grid, dim3(256), 0, ctx->stream, (int)g.M, (int)g.N,
+                     (int)g.K, g.A, g.transA ? g.lda : 1, g.transA ? 1 : g.lda, g.B,
+                     g.transB ? g.ldb : 1, g.transB ? 1 : g.ldb, g.alpha, g.beta, g.C, g.ldc);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    lra_set_error("direct gemm launch: %s", hipGetErrorString(e));
+    return LRA_E_HIP;
+  }
+  return LRA_OK;
+}
+
 // A short-K product with a tall C (the blocked QR's X -= V W and its like): in FP64 on
-// gemm_short_k_kernel.  The low precisions form the transposed product C' = op(B)' op(A)' stored
+// gemm_direct_kernel.  The low precisions form the transposed product C' = op(B)' op(A)' stored
 // transposed: the MFMA output tile then puts 16 consecutive rows of one column of C in 16
 // consecutive lanes, so the read-modify-write of C is coalesced.  One K-range, the general
 // kernel's configuration for the swapped shape.
@@ -1102,18 +1136,7 @@ bool ct_ok(const GemmArgs& g) {
 }
 
 int run_ct(lra_ctx* ctx, const GemmArgs& g) {
-  if (g.prec == LRA_PREC_F64 && g.K >= 1) {
-    const dim3 grid((unsigned)((g.M + 63) / 64), (unsigned)((g.N + 63) / 64));
-    hipLaunchKernelGGL(gemm_short_k_kernel, grid, dim3(256), 0, ctx->stream, (int)g.M, (int)g.N,
-                       (int)g.K, g.A, g.transA ? g.lda : 1, g.transA ? 1 : g.lda, g.B,
-                       g.transB ? g.ldb : 1, g.transB ? 1 : g.ldb, g.alpha, g.beta, g.C, g.ldc);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-      lra_set_error("short-K gemm launch: %s", hipGetErrorString(e));
-      return LRA_E_HIP;
-    }
-    return LRA_OK;
-  }
+  if (g.prec == LRA_PREC_F64 && g.K >= 1) return run_direct(ctx, g);
   GemmArgs s = g;
   s.M = g.N; s.N = g.M;
   s.A = g.B; s.lda = g.ldb; s.transA = !g.transB;
@@ -1154,6 +1177,7 @@ int lra_gemm(lra_ctx* ctx, const GemmArgs& g) {
   if (tn_skinny_ok(g)) return run_tn_skinny(ctx, g);
   if (ct_ok(g)) return run_ct(ctx, g);
   if (narrow_ok(g)) return run_narrow(ctx, g);
+  if (direct_ok(g)) return run_direct(ctx, g);
   TuneKey key{g.prec, g.transA, g.transB, bucket_m(g.M), bucket(g.N), bucket(g.K)};
   TuneVal choice;
   bool have = false;

@@ -275,7 +275,10 @@ def test_sketch_gemm_f32_kc_configs(gpu, monkeypatch, cfg, M, N, K):
 @pytest.mark.parametrize("M,N,K,beta", [
     (1, 1, 1, 0.0), (31, 16, 15, 0.5), (32, 17, 16, 0.0), (33, 64, 65, -2.0), (300, 65, 129, 0.0),
     (65, 1, 4099, 0.0), (129, 256, 1000, 1.0), (20, 33, 8192, 1.0), (2049, 5, 63, 0.0),
-    (70, 130, 2049, 0.0)])
+    (70, 130, 2049, 0.0),
+    # more than 256 columns: operands straight to the MFMAs (gemm_direct_kernel)
+    (70, 300, 231, 0.0), (129, 257, 512, -1.0), (33, 400, 17, 2.0), (1, 600, 1, 0.0),
+    (4100, 511, 16, 1.0), (513, 300, 513, 0.0)])
 def test_dgemm_narrow(gpu, ta, tb, M, N, K, beta):
     """Products with few columns, every storage order, odd offsets and leading dimensions, against
     float64 numpy: sums of K terms in any order differ by at most K eps |a||b| a term."""
