@@ -9,8 +9,7 @@
 // Here: one workgroup per column of A streams X through LDS in slabs of 2*QC columns packed
 // as QC complex sequences, transforms them with an in-place radix-2 FFT (power-of-two l) or a
 // direct DFT (other l), unpacks the two real spectra and accumulates every output frequency in
-// registers.  A is read exactly once (HBM-bound).  Shapes whose transform is compute-bound go
-// to the MFMA GEMM with the SRFT's matrix instead (srft_dense).
+// registers.  A is read exactly once (HBM-bound).
 //
 // Random subset (src/sketch.jl:248-257): B[i,:] = op(A)[r[i],:].
 // Sparse Gaussian (src/sketch.jl:571-589): output row i sums p_i = fld(m-i,ell)+1 rows of op(A)
@@ -19,7 +18,6 @@
 #include "lra_internal.h"
 
 #include <algorithm>
-#include <cstdlib>
 
 namespace {
 
@@ -440,32 +438,6 @@ __global__ void srft_sign_bits_kernel(i64 P, const double* __restrict__ d, uint3
 // sign masks up to 65536 rows (8 KB): the kernel's LDS stays within two workgroups per CU
 constexpr i64 kSignRows = 65536;
 
-// The SRFT's matrix, transposed and for rows t0 .. t0 + rows - 1 of the operand:
-// W[t + slot ldw] = d[t] cos(2 pi f t / m) for an even slot and -d[t] sin(2 pi f t / m) for the
-// odd one after it, f = idx[slot & ~1] - 1.  A thread steps f t mod m exactly (integers).
-constexpr int kPhiRows = 4;  // rows per thread
-__global__ __launch_bounds__(256) void srft_phi_kernel(i64 t0, i64 rows, i64 m,
-                                                       const double* __restrict__ d,
-                                                       const i64* __restrict__ idx, int ell,
-                                                       double* __restrict__ W, i64 ldw) {
-  const int slot = 2 * (int)blockIdx.y;
-  const i64 f = idx[slot] - 1;
-  i64 r = (i64)blockIdx.x * (256 * kPhiRows) + threadIdx.x;
-  i64 e = (i64)(((uint64_t)f * (uint64_t)(t0 + r)) % (uint64_t)m);
-  const i64 step = (f * 256) % m;
-#pragma unroll
-  for (int u = 0; u < kPhiRows; ++u, r += 256) {
-    if (r >= rows) return;
-    double sn, cs;
-    sincospi(-2.0 * (double)e / (double)m, &sn, &cs);
-    const double dt = d[t0 + r];
-    W[r + (i64)slot * ldw] = dt * cs;
-    if (slot + 1 < ell) W[r + (i64)(slot + 1) * ldw] = dt * sn;
-    e += step;
-    if (e >= m) e -= m;
-  }
-}
-
 // B[i, j] = A[r[i]-1, j]
 __global__ void subset_kernel(i64 n, const double* A, i64 lda, int ell, const i64* r, double* B,
                               i64 ldb) {
@@ -548,63 +520,6 @@ static int op_matrix(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i64 l
   return LRA_OK;
 }
 
-// The SRFT as a product with its own ell x P matrix on the MFMA GEMM, for the shapes whose
-// transform is slower: 2 ell P Q flops on the matrix cores (bound by them, about 50 TFLOP/s)
-// against l P Q scalar multiply-adds of a direct DFT of length l, or the nslots P Q / l twiddled
-// sums that a short l leaves to the accumulation.  The matrix is formed in chunks of at most 16384 rows
-// (at order 310 a 41 MB chunk, read back from the last-level cache), and each chunk's product
-// adds to B, which keeps the sums as exact as the transform's: relative error against
-// numpy's FFT 1.6e-15 on 65000 x 4000 at order 310, the transform 1.6e-15.
-// Measured, transform -> product: 65000 x 4000 at order 310 (l = 260) 63.9 -> 3.0 ms, 60000 x
-// 3000 (l = 300) 50.2 -> 2.7 ms, 32008 x 2000 (l = 8) 2.39 -> 0.85 ms, 4099 x 512 at order 50
-// (l = 1) 463 -> 63 us, 32288 x 2000 at order 40 (l = 32) 378 -> 221 us.
-// LRA_E_ALLOC: the workspace does not fit the budget and nothing was done.
-static int srft_dense(lra_ctx* c, i64 P, i64 Q, const double* X, i64 ldx, const double* d,
-                      const i64* idx, i64 ell, double* B, i64 ldb) {
-  // equal chunks of an even number of rows: every product is of one shape
-  const i64 nch = (P + 16383) / 16384;
-  const i64 ldw = ((P + nch - 1) / nch + 1) / 2 * 2, rows = std::min(P, ldw);
-  double* W = nullptr;
-  LRA_CHECK(lra_wsT(c, WS_OMEGA, (size_t)ldw * ell, &W));
-  for (i64 t0 = 0; t0 < P; t0 += rows) {
-    const i64 kr = std::min(rows, P - t0);
-    hipLaunchKernelGGL(srft_phi_kernel,
-                       dim3((unsigned)((kr + 256 * kPhiRows - 1) / (256 * kPhiRows)),
-                            (unsigned)((ell + 1) / 2)),
-                       dim3(256), 0, c->stream, t0, kr, P, d, idx, (int)ell, W, ldw);
-    LRA_LAUNCH_CHECK("srft matrix");
-    GemmArgs g;
-    g.M = ell; g.N = Q; g.K = kr; g.alpha = 1.0; g.beta = t0 == 0 ? 0.0 : 1.0;
-    g.A = W; g.lda = ldw; g.transA = 1; g.B = X + t0; g.ldb = ldx; g.transB = 0;
-    g.C = B; g.ldc = ldb; g.bgather = nullptr; g.prec = LRA_PREC_F64;
-    LRA_CHECK(lra_gemm(c, g));
-  }
-  return LRA_OK;
-}
-
-// Where srft_dense is the faster form (both sides measured with the launches around them):
-//   - l not a power of two: the transform is a direct DFT, l P Q multiply-adds.  200 x 100 at
-//     order 40 (l = 40, 0.8 M) takes 46 us by the DFT and 60 as a product, 1000 x 300 at order
-//     72 (l = 50, 15 M) 66 and 53: the line is 4 M.
-//   - l <= 8 (or any l of a large product, which those always are): the accumulation dominates
-//     and grows with ell P Q.  1048 x 1024 at order 40 (43 M) 39 us and 49, 4099 x 512 at order
-//     50 (105 M) 463 and 63: the line is 64 M.
-//   - l = 16 and 32 on large operands: the slab's two short passes hide little of its load
-//     latency, 392 and 378 us for 32000 x 2000 at order 40 against 222; at order 310 the
-//     transform is ahead (654 and 459 against 790).  The products cross at orders about 160
-//     (l = 16) and 120 (l = 32); 1024 x 1024 at order 40 (42 M) is 40 us and 48.
-//   - l = 64, 128, 256 and longer powers of two stay transforms (289 us against 800 at 64).
-// LRA_SRFT_DENSE=0 or 1 forces either form (1: every shape).
-static bool srft_dense_wins(i64 P, i64 Q, i64 ell, i64 l, bool pow2) {
-  if (const char* f = getenv("LRA_SRFT_DENSE")) return f[0] == '1';
-  const double size = (double)P * (double)Q;
-  if (!pow2) return (double)l * size >= 4e6 || (double)ell * size >= 6.4e7;
-  if (l <= 8) return (double)ell * size >= 6.4e7;
-  if (l == 16) return ell <= 160 && (double)ell * size >= 2.5e8;
-  if (l == 32) return ell <= 120 && (double)ell * size >= 2.5e8;
-  return false;
-}
-
 int lra_sketch_srft_impl(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i64 lda,
                          i64 ell, const double* d, const i64* idx, uint64_t seed,
                          uint64_t stream_id, double* B, i64 ldb) {
@@ -638,10 +553,6 @@ int lra_sketch_srft_impl(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i
   while (P % l) --l;
   const i64 mm = P / l;
   const bool pow2 = (l & (l - 1)) == 0;
-  if (srft_dense_wins(P, Q, ell, l, pow2)) {
-    const int ds = srft_dense(c, P, Q, X, ldx, d, idx, ell, B, ldb);
-    if (ds != LRA_E_ALLOC) return ds;  // (a budget without room for the matrix: the transforms)
-  }
   if (pow2 && ell <= 2048) {
     // two register passes for power-of-two l <= 256
     switch (l) {

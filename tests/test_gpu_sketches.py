@@ -153,46 +153,3 @@ def test_mixed_above_floor_refined(gpu, prec):
     e64, emx = err(V), err(Vm)
     assert abs(V.k - Vm.k) <= 3
     assert emx <= 10 * e64, (emx, e64)
-
-
-@pytest.mark.parametrize("m,n,ell,trans", [
-    (200, 7, 40, "n"),       # l = 40, one chunk
-    (1023, 65, 33, "n"),     # odd order (the last slot is Re only), odd rows
-    (521, 64, 40, "c"),      # transposed operand, prime column count: l = 1
-    (257, 33, 1, "n"),       # one output row
-    (16384, 5, 310, "n"),    # exactly one chunk of rows
-    (16385, 6, 24, "n"),     # one row beyond the first chunk
-    (33000, 3, 310, "n"),    # three chunks, the last one short
-    (64, 40, 64, "n"),       # order = rows
-])
-def test_srft_product_form(gpu, monkeypatch, m, n, ell, trans):
-    """The SRFT as a product with its matrix (forced) against the transform kernels (forced) and
-    numpy's FFT, with a padded leading dimension and a general diagonal.  A sum of m terms in
-    any order is within m eps |d||x| of the exact one; its rounding is a random walk, so the
-    bound is 8 sqrt(m) eps times the column's norm."""
-    import torch
-    rng = np.random.default_rng(m + ell)
-    rows, cols = (m, n) if trans == "n" else (n, m)
-    A = np.asfortranarray(rng.standard_normal((rows, cols)))
-    d = rng.standard_normal(m)
-    idx = rng.integers(1, m + 1, size=ell)
-    lda = rows + 3
-    Ad = torch.zeros((cols, lda), dtype=torch.float64, device="cuda")
-    Ad[:, :rows] = torch.from_numpy(A.T.copy()).cuda()
-    dd, di = torch.from_numpy(d).cuda(), torch.from_numpy(idx).cuda()
-    L, ctx = gpu._lib.load(), gpu.context()
-    got = {}
-    for form in ("0", "1"):
-        monkeypatch.setenv("LRA_SRFT_DENSE", form)
-        B = gpu.empty_colmajor(ell, n)
-        gpu.check(L.lra_sketch_srft(ctx.h, 0 if trans == "n" else 1, rows, cols, Ad.data_ptr(),
-                                    lda, ell, dd.data_ptr(), di.data_ptr(), 0, 0, B.data_ptr(),
-                                    ell), "srft")
-        got[form] = host(B)
-    X = d[:, None] * (A if trans == "n" else A.T)
-    F = np.fft.fft(X, axis=0)[idx[0::2] - 1]
-    E = np.empty((ell, n))
-    E[0::2], E[1::2] = F.real, F.imag[:ell // 2]
-    bound = 8 * np.sqrt(m) * EPS * np.linalg.norm(X, axis=0)[None, :]
-    assert (np.abs(got["1"] - E) <= bound).all()
-    assert (np.abs(got["1"] - got["0"]) <= 2 * bound).all()
