@@ -19,6 +19,15 @@
 
 #include <algorithm>
 
+#define LRA_LAUNCH_CHECK(what)                                                          \
+  do {                                                                                  \
+    hipError_t _e = hipGetLastError();                                                  \
+    if (_e != hipSuccess) {                                                             \
+      lra_set_error("%s launch: %s", what, hipGetErrorString(_e));                      \
+      return LRA_E_HIP;                                                                 \
+    }                                                                                   \
+  } while (0)
+
 namespace {
 
 struct cplx {
@@ -158,6 +167,265 @@ __global__ __launch_bounds__(SRFT_THREADS) void srft_kernel(
     y[2 * s] = acc[u].re;
     if (2 * s + 1 < ell) y[2 * s + 1] = acc[u].im;
   }
+}
+
+// The same transform for an l that is no power of two, in two kernels with srft_kernel's
+// operations in srft_kernel's order, so with its bits: srft_dft_kernel forms the length-l spectra
+// at the frequencies (mod l) that some slot asks for, srft_slots_kernel runs the sums over q.
+// srft_kernel spends its time on index arithmetic and LDS reads, a 64-bit remainder and two reads
+// for one complex product; here a wave holds 64 packed column pairs in its lanes and 8 frequency
+// pairs {f, l - f} in registers, the twiddles come through scalar loads, and what is left is
+// bound by the FP64 vector units (10 instructions for a pair's two complex products): 65000 x 4000 at order 310
+// (l = 260), within the rank-300 ID of 65000 x 4000, 65.7 -> 8.2 ms.
+//
+// Frequencies come in pairs: the spectra of the two packed columns at l - f are the conjugates
+// of those at f.  plist[0..np): the pairs asked for (l < 2048, so at most 1024); slot[s]: its
+// pair, with bit 30 for the conjugate; tw[j] = e^{-2 pi i j / l}; step[s] = e^{-2 pi i f / m};
+// start[b * nslots + s]: the power at the b-th group of 2 qc columns, where srft_kernel also
+// starts anew.
+constexpr int kConj = 1 << 30;
+
+__global__ __launch_bounds__(1024) void srft_plan_kernel(i64 m, int l, int nslots,
+                                                         const i64* __restrict__ idx, int* np,
+                                                         int* plist, int* slot, cplx* tw,
+                                                         cplx* step) {
+  __shared__ int used[1024], wave[16];
+  const int tid = threadIdx.x;
+  used[tid] = 0;
+  __syncthreads();
+  int pr = 0, cj = 0;
+  if (tid < nslots) {
+    const i64 f = idx[2 * tid] - 1;
+    int r = (int)(f % l);
+    r = r < 0 ? r + l : r;
+    cj = r > l - r;
+    pr = cj ? l - r : r;
+    used[pr] = 1;
+    double sn, cs;
+    sincospi(-2.0 * (double)f / (double)m, &sn, &cs);
+    step[tid] = {cs, sn};
+  }
+  __syncthreads();
+  const bool in = used[tid] != 0;
+  const unsigned long long mask = __ballot(in);
+  if ((tid & 63) == 0) wave[tid >> 6] = __popcll(mask);
+  __syncthreads();
+  int k = __popcll(mask & ((1ull << (tid & 63)) - 1)), n = 0;
+  for (int i = 0; i < 16; ++i) {
+    if (i < tid >> 6) k += wave[i];
+    n += wave[i];
+  }
+  if (in) {
+    plist[k] = tid;
+    used[tid] = k;
+  }
+  if (tid == 0) *np = n;
+  __syncthreads();
+  if (tid < nslots) slot[tid] = used[pr] | (cj ? kConj : 0);
+  for (int j = tid; j < l; j += 1024) {
+    const int h = j <= l / 2 ? j : l - j;
+    double sn, cs;
+    sincospi(-2.0 * (double)h / (double)l, &sn, &cs);
+    tw[j] = {cs, j <= l / 2 ? sn : -sn};
+  }
+}
+
+__global__ __launch_bounds__(256) void srft_start_kernel(i64 m, i64 groups, int qc, int nslots,
+                                                         const i64* __restrict__ idx,
+                                                         cplx* start) {
+  const i64 e = (i64)blockIdx.x * 256 + threadIdx.x;
+  if (e >= groups * nslots) return;
+  const i64 f = idx[2 * (e % nslots)] - 1, q0 = e / nslots * 2 * qc;
+  const i64 e0 = (f * (q0 % m)) % m;
+  double sn, cs;
+  sincospi(-2.0 * (double)e0 / (double)m, &sn, &cs);
+  start[e] = {cs, sn};
+}
+
+// X[(column, c)][pair] = {X1, X2}: the spectra of columns 2c and 2c + 1 of the l x mm reshape.
+// 256 (column, c) a workgroup; the workgroups of one such range are 8 apart, on one XCD, and
+// share what they read of A in its L2.
+template <int NP>
+__global__ __launch_bounds__(256) void srft_dft_kernel(
+    i64 m, const double* __restrict__ A, i64 lda, int l, i64 mm, i64 cpc, i64 total, int ntile,
+    const double* __restrict__ d, const int* __restrict__ np, const int* __restrict__ plist,
+    const cplx* __restrict__ tw, int pmax, cplx* __restrict__ X) {
+  const int b8 = blockIdx.x >> 3, tile = b8 % ntile;
+  const i64 e = ((i64)(b8 / ntile) * 8 + (blockIdx.x & 7)) * 256 + threadIdx.x;
+  const int count = *np;
+  if (tile * NP >= count || e - threadIdx.x >= total) return;
+  const i64 ec = e < total ? e : total - 1;
+  const i64 col = ec / cpc, q = 2 * (ec - col * cpc);
+  const double* x = A + col * lda;
+  const bool both = q + 1 < mm;
+  const unsigned lb = 16u * (unsigned)l;  // the twiddles' byte offsets, modulo l entries
+  unsigned fb[NP], jb[NP];
+  cplx a[NP], b[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    fb[i] = 16u * (unsigned)plist[min(tile * NP + i, count - 1)];
+    jb[i] = 0;
+    a[i] = b[i] = {0.0, 0.0};
+  }
+  constexpr int PF = 4;
+  double x0[PF], x1[PF], d0[PF], d1[PF];
+  auto load = [&](int p, int u) {
+    const i64 t = (i64)min(p, l - 1) * mm + q, t1 = both ? t + 1 : t;
+    x0[u] = x[t];
+    x1[u] = x[t1];
+    d0[u] = d[t];
+    d1[u] = d[t1];
+  };
+#pragma unroll
+  for (int u = 0; u < PF; ++u) load(u, u);
+  for (int p0 = 0; p0 < l; p0 += PF) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      if (p0 + u < l) {
+        const cplx z = {d0[u] * x0[u], both ? d1[u] * x1[u] : 0.0};
+        load(p0 + u + PF, u);
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          // (the twiddle at l - f is this one's conjugate, bit for bit)
+          const cplx w = *(const cplx*)((const char*)tw + jb[i]);
+          const double ii = z.im * w.im, ir = z.im * w.re;
+          a[i].re += fma(z.re, w.re, -ii);
+          a[i].im += fma(z.re, w.im, ir);
+          b[i].re += fma(z.re, w.re, ii);
+          b[i].im += fma(z.re, -w.im, ir);
+          const unsigned t = jb[i] + fb[i];
+          jb[i] = min(t, t - lb);  // (t - lb wraps below lb)
+        }
+      }
+    }
+  }
+  if (e >= total) return;
+  cplx* out = X + ((size_t)e * pmax + (size_t)tile * NP) * 2;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    if (tile * NP + i >= count) continue;
+    out[2 * i] = {0.5 * (a[i].re + b[i].re), 0.5 * (a[i].im - b[i].im)};
+    out[2 * i + 1] = {0.5 * (a[i].im + b[i].im), -0.5 * (a[i].re - b[i].re)};
+  }
+}
+
+// cmul as srft_kernel has it compiled: which product of a part is rounded first is fixed here.
+__device__ __forceinline__ cplx cmul_fixed(cplx a, cplx b) {
+  return {fma(a.re, b.re, -(a.im * b.im)), fma(a.im, b.re, a.re * b.im)};
+}
+
+// One thread a slot and NC columns of A: the powers of w, a serial chain, serve NC columns.
+template <int NC>
+__global__ __launch_bounds__(256) void srft_slots_kernel(
+    i64 mm, i64 cpc, i64 cols, int qc, int nslots, const int* __restrict__ slot,
+    const cplx* __restrict__ step, const cplx* __restrict__ start, int pmax,
+    const cplx* __restrict__ X, int ell, double* __restrict__ B, i64 ldb) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= nslots) return;
+  const i64 c0 = (i64)blockIdx.y * NC;
+  const cplx* xs[NC];
+  cplx acc[NC];
+  const double sg = slot[s] & kConj ? -1.0 : 1.0;
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    xs[k] = X + ((size_t)min(c0 + k, cols - 1) * cpc * pmax + (slot[s] & ~kConj)) * 2;
+    acc[k] = {0.0, 0.0};
+  }
+  const cplx ws = step[s];
+  cplx wq = {1.0, 0.0};
+  i64 g = 0;
+  int left = 0;
+  for (i64 c = 0; c < cpc; ++c) {
+    if (left == 0) {
+      wq = start[g * nslots + s];
+      ++g;
+      left = qc;
+    }
+    --left;
+    const cplx w1 = cmul_fixed(wq, ws);
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const cplx* xc = xs[k] + (size_t)c * pmax * 2;
+      const cplx x1 = {xc[0].re, sg * xc[0].im}, x2 = {xc[1].re, sg * xc[1].im};
+      cplx t = cmul_fixed(wq, x1);
+      acc[k].re += t.re;
+      acc[k].im += t.im;
+      if (2 * c + 1 < mm) {
+        t = cmul_fixed(w1, x2);
+        acc[k].re += t.re;
+        acc[k].im += t.im;
+      }
+    }
+    wq = cmul_fixed(w1, ws);
+  }
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    if (c0 + k >= cols) continue;
+    double* y = B + (c0 + k) * ldb;
+    y[2 * s] = acc[k].re;
+    if (2 * s + 1 < ell) y[2 * s + 1] = acc[k].im;
+  }
+}
+
+// Where the two kernels take over from srft_kernel (us): l = 260 of 65000 x 4000 63900 -> 7500, l =
+// 80 of 30000 x 3300 5610 -> 1630, l = 24 of 24216 x 500 534 -> 314, l = 20 of 20180 x 50 413 ->
+// 226; at l = 12 of 12108 x 50 they are even, and for a smaller l, where the sums over q are the
+// work, srft_kernel is ahead (l = 9 of 45027 x 3000 3400, two kernels 7200).  Below 4 M complex
+// products the extra launches cost more than they give (200 x 100 at l = 40: 42 and 46, 1000 x
+// 300 at l = 50 64 and 55).
+bool srft_split(i64 l, i64 P, i64 Q) {
+  if (const char* e = getenv("LRA_SRFT_SPLIT")) return e[0] != '0';
+  return l >= 16 && (double)l * (double)P * (double)Q >= 4e6;
+}
+
+// LRA_E_ALLOC: the workspace does not fit the budget and nothing was done.
+int srft_two_kernels(lra_ctx* c, i64 Q, i64 P, const double* X, i64 ldx, int l, i64 mm, int qc,
+                     const double* d, const i64* idx, int ell, double* B, i64 ldb) {
+  const int nslots = (ell + 1) / 2, pmax = std::min(l / 2 + 1, nslots);
+  const i64 cpc = (mm + 1) / 2, groups = (cpc + qc - 1) / qc;
+  // the spectra of as many columns as fit 256 MB at a time
+  const i64 percol = cpc * pmax * 32;
+  const i64 chunk = std::min(std::min<i64>(Q, 131072), std::max<i64>(1, (256ll << 20) / percol));
+  size_t at = 0;
+  auto take = [&](size_t n) { const size_t o = at; at += (n + 255) & ~(size_t)255; return o; };
+  const size_t o_np = take(4), o_pl = take(4 * (size_t)(l / 2 + 1)), o_sl = take(4 * (size_t)nslots),
+               o_tw = take(16 * (size_t)l), o_st = take(16 * (size_t)nslots),
+               o_gr = take(16 * (size_t)(groups * nslots)), o_x = take((size_t)(chunk * percol));
+  char* w = nullptr;
+  LRA_CHECK(lra_wsT(c, WS_SRFT, at, &w));
+  int* np = (int*)(w + o_np);
+  int* plist = (int*)(w + o_pl);
+  int* slot = (int*)(w + o_sl);
+  cplx *tw = (cplx*)(w + o_tw), *step = (cplx*)(w + o_st), *start = (cplx*)(w + o_gr),
+       *spec = (cplx*)(w + o_x);
+  hipLaunchKernelGGL(srft_plan_kernel, dim3(1), dim3(1024), 0, c->stream, P, l, nslots, idx, np,
+                     plist, slot, tw, step);
+  hipLaunchKernelGGL(srft_start_kernel, dim3((unsigned)((groups * nslots + 255) / 256)), dim3(256),
+                     0, c->stream, P, groups, qc, nslots, idx, start);
+  for (i64 j = 0; j < Q; j += chunk) {
+    const i64 cols = std::min(chunk, Q - j), total = cols * cpc;
+    const int ntile = (pmax + (pmax > 4 ? 7 : 1)) / (pmax > 4 ? 8 : 2);
+    const i64 ranges = (total + 255) / 256;
+    const unsigned grid = (unsigned)((ranges + 7) / 8 * 8 * ntile);
+    if (pmax > 4)
+      hipLaunchKernelGGL(srft_dft_kernel<8>, dim3(grid), dim3(256), 0, c->stream, P, X + j * ldx,
+                         ldx, l, mm, cpc, total, ntile, d, np, plist, tw, pmax, spec);
+    else
+      hipLaunchKernelGGL(srft_dft_kernel<2>, dim3(grid), dim3(256), 0, c->stream, P, X + j * ldx,
+                         ldx, l, mm, cpc, total, ntile, d, np, plist, tw, pmax, spec);
+    const int bt = nslots > 128 ? 256 : nslots > 64 ? 128 : 64;
+    const unsigned gx = (unsigned)((nslots + bt - 1) / bt);
+    if (cols >= 2048)
+      hipLaunchKernelGGL(srft_slots_kernel<4>, dim3(gx, (unsigned)((cols + 3) / 4)), dim3(bt), 0,
+                         c->stream, mm, cpc, cols, qc, nslots, slot, step, start, pmax, spec, ell,
+                         B + j * ldb, ldb);
+    else
+      hipLaunchKernelGGL(srft_slots_kernel<1>, dim3(gx, (unsigned)cols), dim3(bt), 0, c->stream,
+                         mm, cpc, cols, qc, nslots, slot, step, start, pmax, spec, ell,
+                         B + j * ldb, ldb);
+  }
+  LRA_LAUNCH_CHECK("srft in two kernels");
+  return LRA_OK;
 }
 
 // ---- SRFT for power-of-two l <= 256: two register passes of length <= 16 ----------------
@@ -497,15 +765,6 @@ __global__ void sprn_kernel(i64 m, const double* __restrict__ A, i64 lda, int el
 
 }  // namespace
 
-#define LRA_LAUNCH_CHECK(what)                                                          \
-  do {                                                                                  \
-    hipError_t _e = hipGetLastError();                                                  \
-    if (_e != hipSuccess) {                                                             \
-      lra_set_error("%s launch: %s", what, hipGetErrorString(_e));                      \
-      return LRA_E_HIP;                                                                 \
-    }                                                                                   \
-  } while (0)
-
 // op(A) as a column-major P x Q matrix: trans n uses A directly, trans c a transposed copy.
 static int op_matrix(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i64 lda,
                      const double** X, i64* ldx, i64* P, i64* Q) {
@@ -574,6 +833,10 @@ int lra_sketch_srft_impl(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i
   };
   while (qc > 1 && need(qc) > lds_cap) qc >>= 1;
   if (need(qc) > lds_cap) { lra_set_error("srft: l=%lld too large", (long long)l); return LRA_E_UNSUPPORTED; }
+  if (!pow2 && srft_split(l, P, Q)) {
+    const int rc = srft_two_kernels(c, Q, P, X, ldx, (int)l, mm, qc, d, idx, (int)ell, B, ldb);
+    if (rc != LRA_E_ALLOC) return rc;  // (a budget without room for the spectra: srft_kernel)
+  }
   if (need(qc) > 64 * 1024) {
     static std::atomic<uint64_t> lds_set{0};  // per device, set once to the cap need(qc) obeys
     lra_lds_limit_once(lds_set, (const void*)srft_kernel, (int)lds_cap);

@@ -50,6 +50,28 @@ def test_srft_injected_vs_oracle(gpu, orc, m, n, ell):
     assert np.abs(B - ref).max() <= 1e-13 * np.log2(m) * np.abs(F).max()
 
 
+@pytest.mark.parametrize("m,n,ell,free", [
+    (1000, 64, 300, False), (300, 17, 19, True), (300, 17, 17, False), (2047, 3, 2048, False),
+    (31 * 130, 33, 31, True), (24 * 43, 129, 24, False), (48 * 33, 2050, 48, False),
+    (99 * 2, 40, 100, True), (1000, 5, 700, False)])
+@pytest.mark.parametrize("trans", ["n", "c"])
+def test_srft_two_kernels_keep_the_bits(gpu, monkeypatch, m, n, ell, free, trans):
+    """An l that is no power of two (1 or several frequency tiles, odd and even numbers of columns
+    of the reshape, a last group of its powers that is short, a column alone or four a thread):
+    the two kernels against the one, bit for bit.  free: any real d, else signs."""
+    rng = np.random.default_rng(m + n + ell)
+    A = rng.standard_normal((m, n)) * np.exp(8 * rng.standard_normal(n))
+    A = np.asfortranarray(A if trans == "n" else A.T)
+    d = rng.standard_normal(m) if free else np.where(rng.random(m) > 0.5, 1.0, -1.0)
+    idx = rng.integers(1, m + 1, size=ell)
+    idx[:2], idx[2:4] = 1, m
+    out = []
+    for split in ("0", "1"):
+        monkeypatch.setenv("LRA_SRFT_SPLIT", split)
+        out.append(srft_call(gpu, A, ell, d, idx, trans=trans))
+    assert np.array_equal(out[0], out[1])
+
+
 def test_srft_transposed(gpu, orc):
     rng = np.random.default_rng(3)
     A = np.asfortranarray(rng.standard_normal((30, 512)))
