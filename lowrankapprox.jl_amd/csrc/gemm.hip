@@ -1044,7 +1044,15 @@ int run_narrow(lra_ctx* ctx, const GemmArgs& g) {
   kchunk = (kchunk + 63) / 64 * 64;
   splits = (g.K + kchunk - 1) / kchunk;
   double* part = nullptr;
-  if (splits > 1) LRA_CHECK(lra_wsT(ctx, WS_SPLITK, (size_t)(splits * g.M * g.N), &part));
+  if (splits > 1) {
+    const int rc = lra_wsT(ctx, WS_SPLITK, (size_t)(splits * g.M * g.N), &part);
+    if (rc == LRA_E_ALLOC) {  // a budget without room for the partial sums: one range
+      splits = 1;
+      kchunk = (g.K + 63) / 64 * 64;
+    } else if (rc != LRA_OK) {
+      return rc;
+    }
+  }
   const dim3 grid((unsigned)mt, (unsigned)splits, (unsigned)nt);
 #define NARROW(TA, TB, NT)                                                                     \
   hipLaunchKernelGGL((gemm_narrow_kernel<TA, TB, NT>), grid, dim3(256), 0, ctx->stream,        \

@@ -175,8 +175,8 @@ __global__ __launch_bounds__(SRFT_THREADS) void srft_kernel(
 // srft_kernel spends its time on index arithmetic and LDS reads, a 64-bit remainder and two reads
 // for one complex product; here a wave holds 64 packed column pairs in its lanes and 8 frequency
 // pairs {f, l - f} in registers, the twiddles come through scalar loads, and what is left is
-// bound by the FP64 vector units (10 instructions for a pair's two complex products): 65000 x 4000 at order 310
-// (l = 260), within the rank-300 ID of 65000 x 4000, 65.7 -> 8.2 ms.
+// bound by the FP64 vector units (10 instructions for a pair's two complex products): the rank-300
+// ID of 65000 x 4000 (order 310, l = 260) 65.7 -> 8.2 ms, of them 1.7 pivoted QR.
 //
 // Frequencies come in pairs: the spectra of the two packed columns at l - f are the conjugates
 // of those at f.  plist[0..np): the pairs asked for (l < 2048, so at most 1024); slot[s]: its
@@ -378,7 +378,7 @@ bool srft_split(i64 l, i64 P, i64 Q) {
   return l >= 16 && (double)l * (double)P * (double)Q >= 4e6;
 }
 
-// LRA_E_ALLOC: the workspace does not fit the budget and nothing was done.
+// LRA_E_ALLOC: no memory for the workspace, and nothing was done.
 int srft_two_kernels(lra_ctx* c, i64 Q, i64 P, const double* X, i64 ldx, int l, i64 mm, int qc,
                      const double* d, const i64* idx, int ell, double* B, i64 ldb) {
   const int nslots = (ell + 1) / 2, pmax = std::min(l / 2 + 1, nslots);
@@ -833,9 +833,11 @@ int lra_sketch_srft_impl(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i
   };
   while (qc > 1 && need(qc) > lds_cap) qc >>= 1;
   if (need(qc) > lds_cap) { lra_set_error("srft: l=%lld too large", (long long)l); return LRA_E_UNSUPPORTED; }
-  if (!pow2 && srft_split(l, P, Q)) {
+  // (a context with a scratch limit keeps srft_kernel, which needs none: the spectra would take
+  // it from the steps that follow)
+  if (!pow2 && c->hbm_budget == 0 && srft_split(l, P, Q)) {
     const int rc = srft_two_kernels(c, Q, P, X, ldx, (int)l, mm, qc, d, idx, (int)ell, B, ldb);
-    if (rc != LRA_E_ALLOC) return rc;  // (a budget without room for the spectra: srft_kernel)
+    if (rc != LRA_E_ALLOC) return rc;
   }
   if (need(qc) > 64 * 1024) {
     static std::atomic<uint64_t> lds_set{0};  // per device, set once to the cap need(qc) obeys

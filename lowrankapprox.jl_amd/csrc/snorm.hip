@@ -247,9 +247,17 @@ struct Gemv {
         double* y, double beta, const i64* rows = nullptr) const {
     if (m <= 0) return LRA_OK;
     i64 chunk = 0;
-    const i64 nch = gemv_chunks(c, m, nn, most, &chunk);
+    i64 nch = gemv_chunks(c, m, nn, most, &chunk);
     double* p = part;
-    if (!p) LRA_CHECK(lra_wsT(c, WS_X0, (size_t)nch * m, &p));
+    if (!p) {
+      int rc = lra_wsT(c, WS_X0, (size_t)nch * m, &p);
+      if (rc == LRA_E_ALLOC && nch > 1) {  // a budget without room for them: one range
+        nch = 1;
+        chunk = nn;
+        rc = lra_wsT(c, WS_X0, (size_t)m, &p);
+      }
+      LRA_CHECK(rc);
+    }
     if (nn > 0) {
       const dim3 grid((unsigned)((m + GV_ROWS - 1) / GV_ROWS), (unsigned)nch);
       if (m % 2 == 0 && pairs_ok(A, lda, A, m))
