@@ -320,12 +320,13 @@ extern "C" int lra_gaussian_fill(lra_ctx* c, uint64_t seed, uint64_t stream_id, 
 // Gaussian sketch into B; Omega materialised in WS_OMEGA when not injected.
 static int sketch_gaussian_impl(lra_ctx* c, int side, int trans, i64 m, i64 n, const double* A,
                                 i64 lda, i64 ell, const double* omega, uint64_t seed,
-                                uint64_t stream_id, int prec, double* B, i64 ldb) {
+                                uint64_t stream_id, int prec, double* B, i64 ldb, int odd = 1) {
   // op(A) is p x q
   const i64 p = trans == LRA_TRANS_N ? m : n;
   const i64 q = trans == LRA_TRANS_N ? n : m;
   GemmArgs g;
   g.alpha = 1.0; g.beta = 0.0; g.C = B; g.ldc = ldb; g.bgather = nullptr; g.prec = prec;
+  g.odd = odd;
   if (side == LRA_SIDE_LEFT) {
     // B (ell x q) = Omega (ell x p) * op(A)
     g.M = ell; g.N = q; g.K = p;
@@ -362,7 +363,7 @@ static int sketch_gaussian_impl(lra_ctx* c, int side, int trans, i64 m, i64 n, c
 // instead of two short ones, whose M tiles leave the MFMA units part-idle.
 static int sketch_gaussian_left2(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i64 lda,
                                  i64 ell0, i64 ell1, uint64_t seed, uint64_t s0, uint64_t s1,
-                                 double* C) {
+                                 double* C, int odd) {
   const i64 p = trans == LRA_TRANS_N ? m : n;
   const i64 q = trans == LRA_TRANS_N ? n : m;
   const i64 L = ell0 + ell1, ldw = (p + 1) / 2 * 2;
@@ -372,6 +373,7 @@ static int sketch_gaussian_left2(lra_ctx* c, int trans, i64 m, i64 n, const doub
   LRA_CHECK(lra_launch_gaussian_fill_t(c->stream, seed, s1, ell1, p, w + ell0 * ldw, ldw));
   GemmArgs g;
   g.alpha = 1.0; g.beta = 0.0; g.C = C; g.ldc = L; g.bgather = nullptr; g.prec = LRA_PREC_F64;
+  g.odd = odd;
   g.M = L; g.N = q; g.K = p;
   g.A = w; g.lda = ldw; g.transA = 1;
   g.B = A; g.ldb = lda; g.transB = trans == LRA_TRANS_N ? 0 : 1;
@@ -504,7 +506,8 @@ struct SketchFactOut {
 };
 
 int lra_sketch_any(lra_ctx* c, int sketch, int trans, i64 m, i64 n, const double* A, i64 lda,
-                   i64 ell, uint64_t seed, uint64_t stream_id, int prec, double* B, i64 ldb);
+                   i64 ell, uint64_t seed, uint64_t stream_id, int prec, double* B, i64 ldb,
+                   int odd = 1);
 
 static i64 samp_of(const lra_opts* o, i64 x) {
   switch (o->sketch) {
@@ -844,7 +847,7 @@ static int sketchfact_left(lra_ctx* c, int trans, const LraSrc& s, const lra_opt
   SketchFn make = [=](i64 ell, uint64_t stream, int prec, double* B) -> int {
     if (s.op()) LRA_CHECK(op_sketch(c, trans, s, ell, o->seed, stream, B));
     else LRA_CHECK(lra_sketch_any(c, o->sketch, trans, s.m, s.n, s.A, s.lda, ell, o->seed,
-                                  stream, prec, B, ell));
+                                  stream, prec, B, ell, !steady));
     if (niter > 0) LRA_CHECK(power_iterate(c, trans, s, ell, B, niter, herm));
     return LRA_OK;
   };
@@ -852,7 +855,7 @@ static int sketchfact_left(lra_ctx* c, int trans, const LraSrc& s, const lra_opt
   if (!s.op() && o->sketch == LRA_SKETCH_RANDN && niter == 0)
     make2 = [=](i64 ell0, i64 ell1, uint64_t s0, uint64_t s1, double* C) -> int {
       return sketch_gaussian_left2(c, trans, s.m, s.n, s.A, s.lda, ell0, ell1, o->seed, s0, s1,
-                                   C);
+                                   C, !steady);
     };
   return sketchfact_run(c, N, make, o, stream_base, out, !s.op(), make2, steady);
 }
@@ -1216,11 +1219,12 @@ int lra_sketch_sprn_impl(lra_ctx* c, int trans, i64 m, i64 n, const double* A, i
                          uint64_t stream_id, double* B, i64 ldb);
 
 int lra_sketch_any(lra_ctx* c, int sketch, int trans, i64 m, i64 n, const double* A, i64 lda,
-                   i64 ell, uint64_t seed, uint64_t stream_id, int prec, double* B, i64 ldb) {
+                   i64 ell, uint64_t seed, uint64_t stream_id, int prec, double* B, i64 ldb,
+                   int odd) {
   switch (sketch) {
     case LRA_SKETCH_RANDN:
       return sketch_gaussian_impl(c, LRA_SIDE_LEFT, trans, m, n, A, lda, ell, nullptr, seed,
-                                  stream_id, prec, B, ldb);
+                                  stream_id, prec, B, ldb, odd);
     case LRA_SKETCH_SRFT:
       return lra_sketch_srft_impl(c, trans, m, n, A, lda, ell, nullptr, nullptr, seed,
                                   stream_id, B, ldb);

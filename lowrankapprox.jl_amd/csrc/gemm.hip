@@ -305,6 +305,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
   typedef double d2 __attribute__((ext_vector_type(2)));
+  // (8-byte aligned: an odd leading dimension; still one 16-byte load)
+  typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
   // chunk e of a tile -> (row e / KP, k pair e % KP).  Rows past M (columns past N) are read from
   // the last one, and chunks past the tile from its last: unconditional loads, so the wait for
   // one tile's registers leaves the loads of the next in flight.  What they put in the tile
@@ -326,9 +328,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
   auto load_tiles = [&](d2 (&ra)[LA], d2 (&rb)[LB], int tile) {
     const i64 o = (i64)tile * BK;
 #pragma unroll
-    for (int t = 0; t < LA; ++t) ra[t] = *reinterpret_cast<const d2*>(pa[t] + o);
+    for (int t = 0; t < LA; ++t) ra[t] = *reinterpret_cast<const d2u*>(pa[t] + o);
 #pragma unroll
-    for (int t = 0; t < LB; ++t) rb[t] = *reinterpret_cast<const d2*>(pb[t] + o);
+    for (int t = 0; t < LB; ++t) rb[t] = *reinterpret_cast<const d2u*>(pb[t] + o);
   };
   // the last tile when the range does not end on one: k beyond the range is zero
   auto load_tail = [&](d2 (&ra)[LA], d2 (&rb)[LB], int tile) {
@@ -336,7 +338,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
     const i64 o = (i64)tile * BK;
     auto get = [&](const double* src, int c) {
       d2 v = {0.0, 0.0};
-      if (c + 1 < left) v = *reinterpret_cast<const d2*>(src);
+      if (c + 1 < left) v = *reinterpret_cast<const d2u*>(src);
       else if (c < left) v.x = src[0];
       return v;
     };
@@ -759,11 +761,16 @@ constexpr int kNumCfg = 26;
 // rounds' 400 rows (orders 136 + 264) in two M-tiles, 20 and 21 the 112 rows of orders 40 + 72
 // in one.
 bool kc_cfg(int id) { return id >= 5; }
+bool kc_aligned(const GemmArgs& g) {  // k pairs of both operands on 16 bytes
+  return (g.lda % 2) == 0 && (g.ldb % 2) == 0 && ((uintptr_t)g.A % 16) == 0 &&
+         ((uintptr_t)g.B % 16) == 0;
+}
+// g.odd: the sketches take it with operands on 8 bytes too, in tuner classes of their own (order
+// 400 of 5689 x 2048 671 us on the generic tiles, 371 here; order 112 187 and 107).  The products inside the
+// factorizations, and pheig's sketches, keep the generic tiles and their rounding.
 bool kc_ok(const GemmArgs& g) {
   return (g.prec == LRA_PREC_F64 || g.prec == LRA_PREC_F32) && g.transA == 1 && g.transB == 0 &&
-         g.bgather == nullptr &&
-         (g.lda % 2) == 0 && (g.ldb % 2) == 0 && ((uintptr_t)g.A % 16) == 0 &&
-         ((uintptr_t)g.B % 16) == 0;
+         g.bgather == nullptr && (g.odd || kc_aligned(g));
 }
 
 template <int PREC>
@@ -904,10 +911,10 @@ int bk_of(int prec) { return prec == LRA_PREC_F64 ? 16 : 32; }
 // its own, so every product of a class in the process uses one configuration and gives the
 // same bits in any order and under any overlap.
 struct TuneKey {
-  int prec, transA, transB, mb, nb, kb;
+  int prec, transA, transB, mb, nb, kb, odd;
   bool operator<(const TuneKey& o) const {
-    return std::tie(prec, transA, transB, mb, nb, kb) <
-           std::tie(o.prec, o.transA, o.transB, o.mb, o.nb, o.kb);
+    return std::tie(prec, transA, transB, mb, nb, kb, odd) <
+           std::tie(o.prec, o.transA, o.transB, o.mb, o.nb, o.kb, o.odd);
   }
 };
 struct TuneVal { int cfg, splits; };
@@ -1118,7 +1125,7 @@ TuneVal heuristic(const GemmArgs& g, int num_cu) {
 // 1000 (4 M) at K = 231 75 -> 91.
 bool direct_ok(const GemmArgs& g) {
   return g.prec == LRA_PREC_F64 && g.bgather == nullptr && g.K >= 1 && g.K <= 512 &&
-         g.M * g.N <= (1ll << 21) && !kc_ok(g);
+         g.M * g.N <= (1ll << 21) && !(kc_ok(g) && kc_aligned(g));
 }
 
 int run_direct(lra_ctx* ctx, const GemmArgs& g) {
@@ -1186,7 +1193,8 @@ int lra_gemm(lra_ctx* ctx, const GemmArgs& g) {
   if (ct_ok(g)) return run_ct(ctx, g);
   if (narrow_ok(g)) return run_narrow(ctx, g);
   if (direct_ok(g)) return run_direct(ctx, g);
-  TuneKey key{g.prec, g.transA, g.transB, bucket_m(g.M), bucket(g.N), bucket(g.K)};
+  TuneKey key{g.prec, g.transA, g.transB, bucket_m(g.M), bucket(g.N), bucket(g.K),
+              g.odd && !kc_aligned(g)};
   TuneVal choice;
   bool have = false;
   {

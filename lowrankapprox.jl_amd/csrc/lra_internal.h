@@ -296,6 +296,7 @@ struct GemmArgs {
   const i64* bgather;
   int prec;
   int narrow = 0;  // a product with few columns may use its own kernel (the factor products)
+  int odd = 0;  // operands aligned to 8 bytes only may use the k-contiguous kernel (the sketches)
 };
 int lra_gemm(lra_ctx* ctx, const GemmArgs& g);
 

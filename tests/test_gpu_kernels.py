@@ -319,3 +319,24 @@ def test_gemm_kc_k_tiles(gpu, monkeypatch, cfg, prec):
         Om, Ah = host(gpu.gaussian(M, K, 2, 1)), host(A)
         bound = (K + 4) * eps * (np.abs(Om) @ np.abs(Ah))
         assert (np.abs(B - Om @ Ah) <= bound).all(), (M, N, K, splits)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("cfg", [5, 12, 17, 18, 22, 25])
+def test_gemm_kc_operands_on_8_bytes(gpu, monkeypatch, cfg, prec):
+    """The k-contiguous kernel with an odd leading dimension (the columns of A alternate between
+    16- and 8-byte alignment) and with a first element off 16 bytes, odd and even K, one and
+    several K ranges, the last column at the end of its memory: the bound of a K-term sum."""
+    import torch
+    eps = 2.3e-16 if prec == "f64" else 1.2e-7
+    for M, N, K, off, splits in [(3, 5, 1, 0, 1), (17, 130, 15, 0, 1), (40, 33, 33, 0, 1),
+                                 (9, 129, 64, 1, 1), (150, 100, 321, 0, 1), (20, 70, 96, 2, 1),
+                                 (41, 260, 1031, 0, 2), (200, 140, 701, 1, 3)]:
+        rng = np.random.default_rng(M + N + K)
+        big = torch.from_numpy(rng.standard_normal((N, K + off))).cuda()
+        A = big[:, off:].t()
+        monkeypatch.setenv("LRA_GEMM_CFG", f"{cfg}:{splits}")
+        B = host(gpu.sketch("left", "n", A, M, seed=2, stream=1, precision=prec))
+        Om, Ah = host(gpu.gaussian(M, K, 2, 1)), host(A)
+        bound = (K + 4) * eps * (np.abs(Om) @ np.abs(Ah))
+        assert (np.abs(B - Om @ Ah) <= bound).all(), (M, N, K, off, splits)
