@@ -47,7 +47,9 @@ constexpr int QT = 1024;  // threads of every kernel here
 // VPT positions per thread in registers (n <= 1024 VPT), else read three times (VPT = 0).
 // Bound by its chain of dependent loads and barriers: the norms load while thread 0 does the
 // bookkeeping, each wave reduces the waves' maxima itself, and only norms of at least half the
-// largest enter the histogram (256 bins, one wave's scan).
+// largest enter the histogram (256 bins, one wave's scan).  Every wave reads step, length and
+// `done` from the state on entry, so thread 0 keeps their new values until the barrier after the
+// bookkeeping: every wave's entry reads are behind it.
 template <int VPT>
 __global__ __launch_bounds__(QT) void qb_select(int n, int kmax, int nb, int stop_after,
                                                 const double* __restrict__ vn1,
@@ -80,9 +82,9 @@ __global__ __launch_bounds__(QT) void qb_select(int n, int kmax, int nb, int sto
     }
   }
   if (tid < NBIN) hist[tid] = 0;
+  int done = 0, e = b;  // (thread 0's)
   if (tid == 0) {
     const unsigned mask = st->mask;
-    int done = 0, e = b;
     if (b > 0) {
       int j0 = st->j0, jb = st->jb;
       for (int t = 0; t < b && !done; ++t) {
@@ -121,11 +123,6 @@ __global__ __launch_bounds__(QT) void qb_select(int n, int kmax, int nb, int sto
         at[p] = cc;
       }
     }
-    st->s = s0 + e;
-    st->b = 0;
-    st->mask = 0;
-    st->sprev = -1;
-    st->done = done;
     s_done = done;
     s_cnt = 0;
     s_T = NBIN;
@@ -151,6 +148,13 @@ __global__ __launch_bounds__(QT) void qb_select(int n, int kmax, int nb, int sto
     s_mp[wave] = wl < 0 ? INT_MAX : wp;
   }
   __syncthreads();
+  if (tid == 0) {
+    st->s = s0 + e;
+    st->b = 0;
+    st->mask = 0;
+    st->sprev = -1;
+    st->done = done;
+  }
   if (s_done) return;
   const double lv = lane < NW ? s_mx[lane] : -1.0;
   const int lp = lane < NW ? s_mp[lane] : INT_MAX;

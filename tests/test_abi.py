@@ -84,3 +84,17 @@ def test_no_gpu_means_loud_failure(lra):
         pytest.skip("GPU present")
     with pytest.raises(lra.LraError):
         lra.idfact(np.eye(4))
+
+
+def test_candidate_selection_stores_its_state_after_the_barrier():
+    """qb_select (qrcp_block.hip): every wave reads `done`, `s` and `b` of the factorization's state
+    on entry, and thread 0 replaces them; no such store may stand before the first barrier, where
+    another wave's reads can still be ahead."""
+    with open(os.path.join(ROOT, "lowrankapprox.jl_amd", "csrc", "qrcp_block.hip")) as f:
+        src = re.sub(r"//[^\n]*", "", f.read())
+    body = src[src.index("void qb_select("):src.index("void qb_pick_kernel(")]
+    entry, rest = body.split("__syncthreads();", 1)
+    store = r"st->(s|b|done)\s*=[^=]"
+    assert {m[1] for m in re.finditer(r"st->(s|b|done)\b", entry)} == {"s", "b", "done"}
+    assert not re.search(store, entry), re.search(store, entry)[0]
+    assert {m[1] for m in re.finditer(store, rest)} == {"s", "b", "done"}

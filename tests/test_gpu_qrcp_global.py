@@ -237,3 +237,23 @@ def test_blocks_nan_column(gpu, monkeypatch):
         got.append((host(p), k))
     assert got[0][1] == got[1][1] == 60
     assert np.array_equal(got[0][0][:60], got[1][0][:60]) and 12 not in got[0][0][:60]
+
+
+@pytest.mark.parametrize("m,n", [(1040, 3758), (700, 9000), (530, 20000)])
+def test_blocks_repeat_their_bits(gpu, monkeypatch, m, n):
+    """Blocks of steps choose the same pivots and give the same bits each time, with 4, 16 and more
+    positions a thread in the selection of their candidates (its norms in registers, or re-read)."""
+    import torch
+    monkeypatch.setenv("LRA_QRCP_GLOBAL", "1")
+    rng = np.random.default_rng(m)
+    B = rng.standard_normal((m, n)) * np.exp(-0.02 * np.arange(m))[:, None]
+    ref = None
+    for _ in range(6):
+        Bd = gpu.to_device(np.asfortranarray(B))
+        p, tau, k = gpu.geqp3_adap(Bd, -1, 0.0, 1e-7, 32)
+        torch.cuda.synchronize()
+        got = (host(p), host(tau)[:k], host(Bd))  # (tau past the rank is not written)
+        ref = ref or got
+        assert k == len(ref[1]) and k > 300
+        for what, a, b in zip(("pivots", "tau", "factors"), got, ref):
+            assert np.array_equal(a, b), (what, np.argwhere(a != b)[:4])
