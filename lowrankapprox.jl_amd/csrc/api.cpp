@@ -209,6 +209,8 @@ int lra_ws(lra_ctx* c, int slot, size_t bytes, void** out) {
     }
     hipError_t e = hipMalloc(&c->ws[slot], want);
     if (e != hipSuccess) {
+      (void)hipGetLastError();  // (else the next launch check, of a caller that goes on without, sees it)
+      c->ws[slot] = nullptr;
       lra_set_error("workspace hipMalloc(%zu): %s", want, hipGetErrorString(e));
       return LRA_E_ALLOC;
     }
@@ -259,6 +261,9 @@ int lra_coop_area(lra_ctx* c, size_t bytes, void** out, bool* uncached) {
     const size_t want = std::max(bytes, (size_t)1 << 20);
     hipError_t e = hipMalloc(&c->coop, want);
     if (e != hipSuccess) {
+      (void)hipGetLastError();
+      c->coop = nullptr;
+      c->coop_size = 0;
       lra_set_error("coop hipMalloc(%zu): %s", want, hipGetErrorString(e));
       return LRA_E_ALLOC;
     }
