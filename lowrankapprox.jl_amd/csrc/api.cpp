@@ -220,6 +220,14 @@ int lra_ws(lra_ctx* c, int slot, size_t bytes, void** out) {
   return LRA_OK;
 }
 
+void lra_ws_release(lra_ctx* c, int slot) {
+  if (!c->ws[slot]) return;
+  (void)hipStreamSynchronize(c->stream);
+  (void)hipFree(c->ws[slot]);
+  c->ws[slot] = nullptr;
+  c->ws_size[slot] = 0;
+}
+
 // Exchange area of the cooperative kernels.  First choice: a fixed 64 MiB of uncached device
 // memory (reads and writes bypass the per-XCD L2, so blocks exchange data without cache
 // write-back/invalidate); it is never freed before the process ends.  Larger requests fall

@@ -139,6 +139,8 @@ inline void lra_lds_limit_once(std::atomic<uint64_t>& done, const void* fn, int 
 }
 int lra_chkopts_public(const lra_opts* o);  // chkopts! (0 or -(bad field))
 int lra_ws(lra_ctx* ctx, int slot, size_t bytes, void** out);
+// waits for the stream and frees the slot (an optional workspace under a scratch limit)
+void lra_ws_release(lra_ctx* ctx, int slot);
 template <class T>
 static inline int lra_wsT(lra_ctx* ctx, int slot, size_t count, T** out) {
   return lra_ws(ctx, slot, count * sizeof(T), (void**)out);

@@ -890,7 +890,7 @@ int lra_qrcp(lra_ctx* ctx, const QrcpCall& q) {
   const bool force_global = fg && fg[0] == '1';
   if ((force_global && q.mode == 0 && q.offset == 0) || !choose_shape(ctx, q.m, q.n, &sh))
     return lra_qrcp_global(ctx, q);
-  // (where a budget has no room for the copy that the HBM path permutes, the grid takes it)
+  // (where there is no room for the copy that the HBM path permutes, the grid takes it)
   if (q.blocks && q.mode == 0 && q.offset == 0 && lra_qrcp_blocks_fit(ctx, q.m, q.n))
     return lra_qrcp_global(ctx, q);
   QrcpDev d = dev_of(ctx, q, sh);

@@ -1395,7 +1395,10 @@ void launch_fused(hipStream_t s0, int s, int s_first, const QrcpCall& q, int las
 
 }  // namespace
 
+// (Not in a context with a scratch limit: the copy of the sketch that the HBM path permutes, which
+// the register-resident grid does without, would be held when the steps that follow need room.)
 bool lra_qrcp_blocks_fit(lra_ctx* c, int m, int n) {
+  if (c->hbm_budget != 0) return false;
   const char *fe = getenv("LRA_QG_FUSED"), *be = getenv("LRA_QG_BLOCK");
   if ((fe && fe[0] == '0') || (be && be[0] == '0') || m > 8192 || n >= (int)F_NONE) return false;
   double* w = nullptr;
@@ -1478,6 +1481,12 @@ int lra_qrcp_global(lra_ctx* c, const QrcpCall& q) {
       // kShort steps on average (many columns of nearly equal norm, or norms outside the
       // blocks' range) single steps run, twice as many each time.
       const char* be = getenv("LRA_QG_BLOCK");
+      // In a context with a scratch limit the blocks' workspace (0.1 MB and 128 bytes a row) goes
+      // back at the end, so that single steps' limits still hold what follows.
+      struct GiveBack {
+        lra_ctx* c;
+        ~GiveBack() { if (c->hbm_budget != 0) lra_ws_release(c, WS_QGB); }
+      } give_back{c};
       double* wb = nullptr;
       const bool block = !(be && be[0] == '0') && lra_wsT(c, WS_QGB, lra_qb_doubles(m), &wb) == LRA_OK;
       if (!block) {

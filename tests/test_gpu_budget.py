@@ -1,7 +1,77 @@
-"""Scratch memory that cannot be had."""
+"""Contexts with a scratch limit (lra_ctx_create's hbm_budget): what succeeded on the paths that
+need the least scratch succeeds under the same limit on the faster ones."""
+import contextlib
+
+import numpy as np
 import pytest
 
+from test_gpu_kernels import host
+
 pytestmark = pytest.mark.gpu
+
+STEP = 32 << 10
+
+
+@contextlib.contextmanager
+def limited(gpu, budget):
+    """The package's context replaced by one with a scratch limit of `budget` bytes."""
+    import torch
+    dev = torch.cuda.current_device()
+    plain = gpu._lib.Context.get(dev)
+    ctx = gpu._lib.Context(dev, budget)
+    gpu._lib.Context._ctx[dev] = ctx
+    try:
+        yield
+        torch.cuda.synchronize()
+    finally:
+        gpu._lib.Context._ctx[dev] = plain
+        ctx.close()
+
+
+def smallest_budget(gpu, call, most=1 << 30):
+    """The smallest limit (to STEP bytes) under which a fresh context runs `call`."""
+    lo, hi = 0, most // STEP
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        try:
+            with limited(gpu, mid * STEP):
+                call()
+            hi = mid
+        except gpu.LraError as e:
+            assert "budget" in str(e), e
+            lo = mid
+    return hi * STEP
+
+
+def spectrum(m, n, fall, seed):
+    """A matrix with singular values exp(-fall i)."""
+    rng = np.random.default_rng(seed)
+    r = min(m, n)
+    U, _ = np.linalg.qr(rng.standard_normal((m, r)))
+    V, _ = np.linalg.qr(rng.standard_normal((n, r)))
+    return (U * np.exp(-fall * np.arange(r))) @ V.T
+
+
+@pytest.mark.parametrize("m,n,fall,rtol,env", [
+    # orders 520 (rejected) and 1032 on the register grid or in blocks, one after the other
+    (1500, 1500, 0.015, 1e-4, {"LRA_QRCP_PAIR": "0"}),
+    (1400, 1300, 0.02, 1e-7, {"LRA_QRCP_GLOBAL": "1"})])  # every round in HBM
+def test_blocks_fit_where_single_steps_did(gpu, monkeypatch, m, n, fall, rtol, env):
+    """The smallest limit that holds a slowly decaying idfact without blocks of pivoted-QR steps
+    holds it with them, and gives the same ID."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    A = gpu.to_device(spectrum(m, n, fall, 5))
+    run = lambda: gpu.idfact(A, rtol=rtol, seed=4)
+    V1 = run()  # (products tuned without a limit)
+    monkeypatch.setenv("LRA_QG_BLOCK", "0")
+    V0 = run()
+    budget = smallest_budget(gpu, run)
+    monkeypatch.delenv("LRA_QG_BLOCK")
+    assert V1.k == V0.k > 500
+    with limited(gpu, budget):
+        V = run()
+    assert V.k == V0.k and np.array_equal(host(V.sk), host(V0.sk))
 
 
 def test_refused_workspace_leaves_no_error(gpu):
