@@ -1044,9 +1044,17 @@ bool narrow_ok(const GemmArgs& g) {
   return g.N <= 64 || g.K <= 2048 || !kc_ok(g);
 }
 
+TuneVal heuristic(const GemmArgs& g, int num_cu);
+
 int run_narrow(lra_ctx* ctx, const GemmArgs& g) {
   const i64 mt = (g.M + 31) / 32, nt = (g.N + 63) / 64, tiles = mt * nt;
   i64 splits = std::max<i64>(1, std::min<i64>((2 * ctx->num_cu + tiles - 1) / tiles, g.K / 128));
+  // a context with a scratch limit: no more partial sums than the tiled kernels would take, or
+  // than the slot holds already, so that what follows finds the room it needs
+  if (ctx->hbm_budget != 0)
+    splits = std::min<i64>(splits, std::max<i64>(heuristic(g, ctx->num_cu).splits,
+                                                 (i64)(ctx->ws_size[WS_SPLITK] / sizeof(double)) /
+                                                     (g.M * g.N)));
   i64 kchunk = (g.K + splits - 1) / splits;
   kchunk = (kchunk + 63) / 64 * 64;
   splits = (g.K + kchunk - 1) / kchunk;

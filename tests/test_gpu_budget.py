@@ -74,6 +74,30 @@ def test_blocks_fit_where_single_steps_did(gpu, monkeypatch, m, n, fall, rtol, e
     assert V.k == V0.k and np.array_equal(host(V.sk), host(V0.sk))
 
 
+def direct_id(gpu):
+    """An ID without a sketch, and the smallest limit that holds it."""
+    B = gpu.to_device(spectrum(700, 900, 0.05, 2))
+    call = lambda: gpu.idfact(B, rtol=1e-9, sketch="none")
+    k = call().k
+    return call, k, smallest_budget(gpu, call)
+
+
+def test_narrow_product_leaves_room(gpu):
+    """A product with few columns whose tiled form takes no scratch (1024 x 64, K = 512, beta = 1)
+    leaves a limited context's room to the call that follows."""
+    import torch
+    call, k, budget = direct_id(gpu)
+    rng = np.random.default_rng(3)
+    A, B, C = (np.asfortranarray(rng.standard_normal(s)) for s in ((1024, 512), (512, 64), (1024, 64)))
+    ref = A @ B + C
+    with limited(gpu, budget):
+        Cd = gpu.to_device(C).clone().t().contiguous().t()
+        gpu.dgemm(A, B, "n", "n", 1.0, Cd, 1.0)
+        assert call().k == k
+    bound = 2.3e-16 * 520 * (np.abs(A) @ np.abs(B) + np.abs(C))
+    assert (np.abs(host(Cd) - ref) <= bound).all()
+
+
 def test_refused_workspace_leaves_no_error(gpu):
     """A workspace that the device cannot give is an error of that call alone."""
     import torch
