@@ -231,6 +231,14 @@ i64 gemv_chunks(const lra_ctx* c, i64 m, i64 n, size_t most, i64* chunk) {
   return n > 0 ? (n + *chunk - 1) / *chunk : 1;
 }
 
+// The number of chunks of at least 256 columns for about four blocks of 256 rows per CU: the partial
+// sums that a caller with little memory has room for (lra_snormdiff_id_noalloc's array, a context
+// with a scratch limit).
+i64 least_chunks(const lra_ctx* c, i64 m, i64 n) {
+  const i64 rt = std::max<i64>(1, (m + 255) / 256);
+  return std::max<i64>(1, std::min<i64>((n + 255) / 256, (4ll * c->num_cu + rt - 1) / rt));
+}
+
 // whether rows (pairs of doubles) of A and x can be read 16 bytes at a time
 bool pairs_ok(const double* A, i64 lda, const double* x, i64 m) {
   return m >= 2 && lda % 2 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)x & 15) == 0;
@@ -359,9 +367,13 @@ struct PowerBufs {
 // The estimate and the stop test are on the device: the host enqueues four steps, then eight
 // at a time, and reads the state after each batch (steps after the stop return at once).  A
 // caller's operator is applied exactly as often as the reference applies it: one step at a time.
-int power_iteration(lra_ctx* c, const Op& o, int isherm, const lra_opts* opts, const double* x0,
+int power_iteration(lra_ctx* c, const Op& op, int isherm, const lra_opts* opts, const double* x0,
                     double* result, const PowerBufs* given = nullptr) {
+  Op o = op;
   const i64 m = o.m, n = o.n;
+  // (what a limited context gives to partial sums it holds from here on: more of them than these
+  // would take the room of the calls that follow)
+  if (!given && c->hbm_budget != 0) o.most = (size_t)std::max<i64>(1, least_chunks(c, m, n) * m);
   double *xn = nullptr, *xm = nullptr, *wk = nullptr;
   if (given) {
     xn = given->xn; xm = given->xm; wk = given->wk;
@@ -513,12 +525,8 @@ extern "C" int lra_snormdiff_id_noalloc(lra_ctx* c, int64_t m, int64_t n, const 
   LRA_ARG(opts != nullptr, 11);
   LRA_ARG(result != nullptr, 13);
   // scratch layout: xn (n) | xm (m) | wk (max(k,1) + 64) | GEMV partial sums, with what is left
-  // (at least the sums of 256-column chunks, about four blocks of 256 rows per CU)
-  auto parts = [&](i64 cols) {
-    const i64 rt = (m + 255) / 256;
-    return std::max<i64>(1, std::min<i64>((cols + 255) / 256, (4ll * c->num_cu + rt - 1) / std::max<i64>(rt, 1)));
-  };
-  const i64 nparts = std::max(parts(n), parts(k));
+  // (at least the sums of `least_chunks`)
+  const i64 nparts = least_chunks(c, m, n);
   const size_t head = (size_t)std::max<i64>(n, 1) + (size_t)std::max<i64>(m, 1) +
                       (size_t)std::max<i64>(k, 1) + 64;
   const size_t need = head + (size_t)nparts * (size_t)m;

@@ -98,6 +98,24 @@ def test_narrow_product_leaves_room(gpu):
     assert (np.abs(host(Cd) - ref) <= bound).all()
 
 
+@pytest.mark.parametrize("m,n", [(600, 40000), (2000, 9000)])
+def test_snorm_leaves_room(gpu, m, n):
+    """snorm under a limit keeps to the partial sums of 256-column chunks, as many as about four
+    blocks of 256 rows per CU ask for: an ID that fits beside them still fits after it."""
+    import torch
+    call, k, budget = direct_id(gpu)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    A = torch.randn((n, m), generator=g, device="cuda", dtype=torch.float64).t()
+    ref = gpu.snorm(A, snorm_niter=4, rtol=0.0)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rt = -(-m // 256)
+    chunks = min(-(-n // 256), -(-4 * cus // rt))
+    with limited(gpu, budget + 8 * (n + m + 65 + chunks * m)):
+        got = gpu.snorm(A, snorm_niter=4, rtol=0.0)
+        assert call().k == k
+    assert abs(got - ref) <= 1e-12 * ref
+
+
 def test_refused_workspace_leaves_no_error(gpu):
     """A workspace that the device cannot give is an error of that call alone."""
     import torch
