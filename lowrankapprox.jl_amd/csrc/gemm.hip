@@ -1095,8 +1095,11 @@ int run_narrow(lra_ctx* ctx, const GemmArgs& g) {
   return LRA_OK;
 }
 
+// Operands on 8 bytes get no more K ranges on the k-contiguous kernel's wider tiles than on the
+// generic ones: the partial sums are scratch that a context may limit.
 void candidates(const GemmArgs& g, int num_cu, std::vector<TuneVal>* out) {
-  const bool kc = kc_ok(g);
+  const bool kc = kc_ok(g), odd = kc && !kc_aligned(g);
+  int generic = 1;
   for (int cfg = 0; cfg < kNumCfg; ++cfg) {
     const Cfg& c = kCfgs[cfg];
     if (kc_cfg(cfg) && !kc) continue;
@@ -1108,6 +1111,8 @@ void candidates(const GemmArgs& g, int num_cu, std::vector<TuneVal>* out) {
     for (int s : {1, 2, 3, 4, 6, 8, 16, 32}) {
       if (s > 1 && tiles * s > 8ll * num_cu) break;
       if (s > 1 && g.K / s < 256) break;
+      if (!kc_cfg(cfg)) generic = std::max(generic, s);
+      else if (odd && s > generic) break;
       out->push_back({cfg, s});
     }
   }

@@ -116,6 +116,19 @@ def test_snorm_leaves_room(gpu, m, n):
     assert abs(got - ref) <= 1e-12 * ref
 
 
+def test_odd_sketch_takes_no_larger_partials(gpu):
+    """The tuner's candidates for a sketch with an odd leading dimension take no more K ranges
+    (their partial sums are the scratch) than the generic tiles': 16 at 531 x 2048, K = 8193."""
+    import torch
+    m, n, order = 8193, 2048, 531
+    g = torch.Generator(device="cuda").manual_seed(2)
+    A = torch.randn((n, m), generator=g, device="cuda", dtype=torch.float64).t()
+    with limited(gpu, 8 * (order * (m + 1) + 16 * order * n) + (1 << 16)):
+        B = host(gpu.sketch("left", "n", A, order, seed=3))
+    Om, Ah = host(gpu.gaussian(order, m, 3, 0)), host(A)
+    assert (np.abs(B - Om @ Ah) <= 2.3e-16 * (m + 4) * (np.abs(Om) @ np.abs(Ah))).all()
+
+
 def test_refused_workspace_leaves_no_error(gpu):
     """A workspace that the device cannot give is an error of that call alone."""
     import torch
