@@ -765,13 +765,17 @@ bool kc_aligned(const GemmArgs& g) {  // k pairs of both operands on 16 bytes
   return (g.lda % 2) == 0 && (g.ldb % 2) == 0 && ((uintptr_t)g.A % 16) == 0 &&
          ((uintptr_t)g.B % 16) == 0;
 }
-// g.odd: the sketches take it with operands on 8 bytes too, in tuner classes of their own (order
+// g.odd: the sketches take it with operands on 8 bytes too (order
 // 400 of 5689 x 2048 671 us on the generic tiles, 371 here; order 112 187 and 107).  The products inside the
 // factorizations, and pheig's sketches, keep the generic tiles and their rounding.
 bool kc_ok(const GemmArgs& g) {
   return (g.prec == LRA_PREC_F64 || g.prec == LRA_PREC_F32) && g.transA == 1 && g.transB == 0 &&
          g.bgather == nullptr && (g.odd || kc_aligned(g));
 }
+// Which kernels a product may take: products of one shape but different classes are tuned apart,
+// since a configuration found for one may not be another's.  0: the generic tiles only, 1: the
+// k-contiguous kernel too, 2: the k-contiguous kernel with operands on 8 bytes.
+int kc_class(const GemmArgs& g) { return !kc_ok(g) ? 0 : kc_aligned(g) ? 1 : 2; }
 
 template <int PREC>
 hipError_t launch_cfg(int id, const GemmDev& d, int blocks, hipStream_t st) {
@@ -911,10 +915,10 @@ int bk_of(int prec) { return prec == LRA_PREC_F64 ? 16 : 32; }
 // its own, so every product of a class in the process uses one configuration and gives the
 // same bits in any order and under any overlap.
 struct TuneKey {
-  int prec, transA, transB, mb, nb, kb, odd;
+  int prec, transA, transB, mb, nb, kb, kc;
   bool operator<(const TuneKey& o) const {
-    return std::tie(prec, transA, transB, mb, nb, kb, odd) <
-           std::tie(o.prec, o.transA, o.transB, o.mb, o.nb, o.kb, o.odd);
+    return std::tie(prec, transA, transB, mb, nb, kb, kc) <
+           std::tie(o.prec, o.transA, o.transB, o.mb, o.nb, o.kb, o.kc);
   }
 };
 struct TuneVal { int cfg, splits; };
@@ -933,6 +937,10 @@ int bucket(i64 x) {  // power-of-two bucket
 // depends on how the order divides into tiles, e.g. 400 rows fill two 208-row tiles but
 // 264 rows fit a 160 x 256 tile better), the power-of-two bucket beyond
 int bucket_m(i64 m) { return m <= 1024 ? (int)((m + 15) / 16) : 64 + bucket(m); }
+
+TuneKey key_of(const GemmArgs& g) {
+  return {g.prec, g.transA, g.transB, bucket_m(g.M), bucket(g.N), bucket(g.K), kc_class(g)};
+}
 
 int prepare(lra_ctx* ctx, const GemmArgs& g, int cfg, int splits, GemmDev* d, int* blocks) {
   const Cfg& c = kCfgs[cfg];
@@ -1098,7 +1106,7 @@ int run_narrow(lra_ctx* ctx, const GemmArgs& g) {
 // Operands on 8 bytes get no more K ranges on the k-contiguous kernel's wider tiles than on the
 // generic ones: the partial sums are scratch that a context may limit.
 void candidates(const GemmArgs& g, int num_cu, std::vector<TuneVal>* out) {
-  const bool kc = kc_ok(g), odd = kc && !kc_aligned(g);
+  const bool kc = kc_ok(g), odd = kc_class(g) == 2;
   int generic = 1;
   for (int cfg = 0; cfg < kNumCfg; ++cfg) {
     const Cfg& c = kCfgs[cfg];
@@ -1206,8 +1214,7 @@ int lra_gemm(lra_ctx* ctx, const GemmArgs& g) {
   if (ct_ok(g)) return run_ct(ctx, g);
   if (narrow_ok(g)) return run_narrow(ctx, g);
   if (direct_ok(g)) return run_direct(ctx, g);
-  TuneKey key{g.prec, g.transA, g.transB, bucket_m(g.M), bucket(g.N), bucket(g.K),
-              g.odd && !kc_aligned(g)};
+  const TuneKey key = key_of(g);
   TuneVal choice;
   bool have = false;
   {
@@ -1285,12 +1292,16 @@ int lra_gemm(lra_ctx* ctx, const GemmArgs& g) {
   return run(ctx, g, choice.cfg, choice.splits);
 }
 
-// Report the configuration chosen for a shape (for the bench's roofline bookkeeping).
+// Report the configuration chosen for a sketch's shape with operands on 16 bytes (for the bench's
+// roofline bookkeeping).  LRA_E_STATE: not tuned yet.
 extern "C" int lra_gemm_choice(int prec, int transA, int transB, int64_t M, int64_t N,
                                int64_t K, int* cfg, int* splits, int* bm, int* bn) {
-  TuneKey key{prec, transA, transB, bucket_m(M), bucket(N), bucket(K)};
+  GemmArgs g{};
+  g.M = M; g.N = N; g.K = K;
+  g.transA = transA; g.transB = transB; g.prec = prec;
+  g.lda = g.ldb = 2;  // (even, as the null pointers: aligned)
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  auto it = g_tune.find(key);
+  auto it = g_tune.find(key_of(g));
   if (it == g_tune.end()) return LRA_E_STATE;
   *cfg = it->second.cfg;
   *splits = it->second.splits;

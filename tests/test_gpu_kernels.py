@@ -340,3 +340,26 @@ def test_gemm_kc_operands_on_8_bytes(gpu, monkeypatch, cfg, prec):
         Om, Ah = host(gpu.gaussian(M, K, 2, 1)), host(A)
         bound = (K + 4) * eps * (np.abs(Om) @ np.abs(Ah))
         assert (np.abs(B - Om @ Ah) <= bound).all(), (M, N, K, off, splits)
+
+
+def test_tuner_classes_by_alignment(gpu):
+    """Products that the k-contiguous kernel takes and products of the same sizes that it does not
+    (an operand off 16 bytes) are tuned apart: neither finds the other's configuration."""
+    import ctypes
+    import torch
+    M, N, K = 300, 700, 1500
+
+    def choice():
+        o = [ctypes.c_int(-1) for _ in range(4)]
+        st = gpu._lib.load().lra_gemm_choice(0, 1, 0, M, N, K, *map(ctypes.byref, o))
+        return st, o[0].value
+
+    rng = np.random.default_rng(4)
+    Ah, Bh = rng.standard_normal((K, M)), rng.standard_normal((K, N))
+    bound = 2.3e-16 * (K + 4) * (np.abs(Ah).T @ np.abs(Bh))
+    for pad, tuned in ((1, False), (2, True)):  # odd, then even leading dimension
+        A, B = (torch.from_numpy(np.pad(X, ((0, pad), (0, 0))).T.copy()).cuda().t()[:K]
+                for X in (Ah, Bh))
+        C = host(gpu.dgemm(A, B, "c", "n"))
+        assert (np.abs(C - Ah.T @ Bh) <= bound).all()
+        assert (choice()[0] == 0) == tuned
