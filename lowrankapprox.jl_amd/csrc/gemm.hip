@@ -1293,13 +1293,14 @@ int lra_gemm(lra_ctx* ctx, const GemmArgs& g) {
 }
 
 // Report the configuration chosen for a sketch's shape with operands on 16 bytes (for the bench's
-// roofline bookkeeping).  LRA_E_STATE: not tuned yet.
+// roofline bookkeeping).  LRA_E_STATE: not tuned yet, or a shape whose kernel is not tuned.
 extern "C" int lra_gemm_choice(int prec, int transA, int transB, int64_t M, int64_t N,
                                int64_t K, int* cfg, int* splits, int* bm, int* bn) {
   GemmArgs g{};
   g.M = M; g.N = N; g.K = K;
   g.transA = transA; g.transB = transB; g.prec = prec;
   g.lda = g.ldb = 2;  // (even, as the null pointers: aligned)
+  if (tn_skinny_ok(g) || ct_ok(g) || direct_ok(g)) return LRA_E_STATE;
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tune.find(key_of(g));
   if (it == g_tune.end()) return LRA_E_STATE;

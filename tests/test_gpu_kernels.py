@@ -363,3 +363,17 @@ def test_tuner_classes_by_alignment(gpu):
         C = host(gpu.dgemm(A, B, "c", "n"))
         assert (np.abs(C - Ah.T @ Bh) <= bound).all()
         assert (choice()[0] == 0) == tuned
+
+
+def test_choice_of_an_untuned_kernel(gpu):
+    """lra_gemm_choice reports no tile for a shape that runs on a kernel without a choice, also where
+    a larger product of its tuner class has one."""
+    import ctypes
+    rng = np.random.default_rng(4)
+    A, B = (np.asfortranarray(rng.standard_normal(s)) for s in ((1000, 300), (300, 4000)))
+    gpu.dgemm(A, B)
+
+    def choice(N):
+        return gpu._lib.load().lra_gemm_choice(0, 0, 0, 1000, N, 300, *(ctypes.byref(ctypes.c_int())
+                                                                       for _ in range(4)))
+    assert choice(4000) == 0 and choice(2060) != 0
