@@ -569,14 +569,16 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
   // The diagonal of R foreseen from a rejected round of order ell and target t, taken to fall
   // geometrically from |R(0,0)| to |R(t-1,t-1)|, where |R(i,i)| stands for sigma_i
   // sqrt(ell - i) (the rows that a Gaussian sketch has left at step i).  A round of order l2 and
-  // target t2 is foreseen to be accepted when its |R(t2-1,t2-1)| is below ptol.  Only
-  // which rounds share a launch depends on it, not what a round gives.  An accepted round that
+  // target t2 is foreseen to be accepted when its |R(t2-1,t2-1)| is below ptol.  It decides which
+  // rounds share a launch (and so a merged product's rounding of their sketches) and which kernel
+  // factors a round, never a round's Omega or its stop rule.  An accepted round that
   // runs alone saves its partner's sketch and the larger grid (rank 100 of 8192 x 8192: 2.85 ->
   // 1.72 ms, rank 180 of 2999 x 2999: 3.56 -> 2.63 ms); one that is rejected after all loses
   // the overlap of the two (about 1.5 ms at orders 264 and 520 of 2999 columns), so the line is
   // where either outcome is as likely.  steady: the caller's results hang on the sketch's
   // rounding (a Hermitian factorization's eigenvectors take their signs from it), which a
-  // round's share of a merged product changes; its rounds pair as their sizes allow.
+  // round's share of a merged product changes; its rounds pair as their sizes allow, and nothing
+  // is foreseen.
   double slope = 0.0, depth = 0.0;  // log fall of sigma per step; log(ptol / |R(0,0)|)
   auto foresee = [&](const i64* hv, i64 ell, i64 t) {
     double r0 = 0.0, rl = 0.0;
@@ -584,7 +586,7 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
     std::memcpy(&rl, &hv[3], sizeof(double));
     const double ptol = std::max(o->atol, o->rtol * r0);
     slope = depth = 0.0;
-    if (steady || t < 2 || !(rl > 0.0) || !(ptol > 0.0) || !(ptol < r0)) return;
+    if (t < 2 || !(rl > 0.0) || !(ptol > 0.0) || !(ptol < r0)) return;
     slope = (std::log(rl / r0) + 0.5 * std::log((double)ell / (double)(ell - t + 1))) / (double)(t - 1);
     depth = std::log(ptol / r0);
   };
@@ -647,7 +649,7 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
         }
         const int st = lra_qrcp_pair(c, qs[0], qs[1]);
         if (st == LRA_OK) {
-          const bool look = targets[1] <= std::min<i64>(ells[1], N);
+          const bool look = !steady && targets[1] <= std::min<i64>(ells[1], N);
           if (look)
             LRA_CHECK(lra_launch_two_diagonals(c->stream, qs[1].A, qs[1].lda, targets[1] - 1,
                                                (double*)(dk + 2)));
@@ -705,8 +707,11 @@ static int sketchfact_run(lra_ctx* c, i64 N, const SketchFn& make, const lra_opt
     LRA_CHECK(lra_qrcp(c, q));
     // with rtol below the floor, a rejected low-precision round also reports |R(0,0)| (the
     // largest column norm) and |R(t-1,t-1)|, t = target: R is written back on every exit; so does
-    // an FP64 round whose successor may pair
-    const bool look = adap && target >= 1 && target <= l && (lowp ? o->rtol < floor : pair_ok);
+    // an FP64 round whose successor may pair by what it foresees (`foresee`; read with the rank,
+    // accepted or not: 4 us of one launch, where a second read of a rejected round's diagonal
+    // costs 20)
+    const bool look = adap && target >= 1 && target <= l &&
+                      (lowp ? o->rtol < floor : pair_ok && !steady);
     if (look) LRA_CHECK(lra_launch_two_diagonals(c->stream, B, ell, target - 1, (double*)(dk + 2)));
     i64 hv[4] = {0, 0, 0, 0};
     LRA_CHECK(read_scalars(c, dk, hv, look ? 4 : 1));
