@@ -27,6 +27,10 @@ inline size_t lra_qb_doubles(int m) {
 }
 QbWork lra_qb_work(double* w, int m);
 
+// Steps a block of that many rows holds: the panel keeps its columns in the registers of one
+// workgroup, at most 36 doubles a thread.
+inline int lra_qb_cap(int rows) { return rows <= 2048 ? 16 : rows <= 3072 ? 12 : rows <= 4096 ? 8 : 4; }
+
 // Selects the candidates of the first block.
 int lra_qb_start(lra_ctx* c, const QrcpCall& q, const QbWork& w, const int* at, double* vn1,
                  const double* diag, FState* st);

@@ -792,7 +792,7 @@ int lra_qb_blocks(lra_ctx* c, const QrcpCall& q, const QbWork& w, int* at, doubl
   const unsigned ga = (unsigned)std::max(1, (n - s - 1 + 15) / 16);
   for (int k = 0; k < count; ++k) {
     hipLaunchKernelGGL(qb_gram, dim3(36), dim3(QT), 0, c->stream, m, q.A, q.lda, w.cand, w.G, st);
-    // the block's columns fill at most 48 doubles a thread (96 of its 128 registers)
+    // (the steps a panel holds: lra_qb_cap)
     if (rows <= QT) launch_panel<1, 16>(c, q, w, at, vn1, vn2, diag, st);
     else if (rows <= 2 * QT) launch_panel<2, 16>(c, q, w, at, vn1, vn2, diag, st);
     else if (rows <= 3 * QT) launch_panel<3, 12>(c, q, w, at, vn1, vn2, diag, st);

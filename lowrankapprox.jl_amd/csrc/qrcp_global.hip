@@ -1395,6 +1395,25 @@ void launch_fused(hipStream_t s0, int s, int s_first, const QrcpCall& q, int las
 
 }  // namespace
 
+// Steps that a block must hold to be ahead of single steps on `rows` x `cols` of trailing matrix.  A
+// block costs 17 us + 21 ns a row (48 us + 15.5 ns beyond 2304 rows, where its apply reads the
+// columns twice) for its selection, Gram matrix and the panel's fixed part, 3.2 us a step, and for
+// the apply 0.8 us a million elements, 3 where its workgroups come in two waves (more than 4096
+// columns), 5.5 from 256 MB on; a single step costs 8.3 us + 2 ns a row, and 1.4 us a million
+// elements up to 4 million, 2.8 beyond (2.0 and 4.2 from 4097 rows, in another form).  Fitted to 300
+// to 8192 rows by 264 to 8000 columns; a tenth on top for the launches of a batch after the end.
+// At falls of 1 and 10% a step a block holds 8 to 16 and 4 to 7 steps, and the two, single and
+// blocks, took us a step: 1040 x 4000 17 and 8, 15; 2056 x 520 13 and 9, 15; 2800 x 1032 17 and 12,
+// 23; 4096 x 264 17 and 20, 22; 8192 x 520, where at most 4 steps fit, 33 and 62, 64; 8192 x 2000 78
+// and 63, 66.
+static double block_steps_needed(int rows, int cols) {
+  const double r = rows, mel = 1e-6 * r * cols, lo = std::min(mel, 4.0), hi = mel - lo;
+  const double block = (rows <= 2304 ? 17.0 + 0.021 * r : 48.0 + 0.0155 * r) +
+                       mel * (mel >= 32.0 ? 5.5 : cols > 4096 ? 3.0 : 0.8);
+  const double single = 8.3 + 0.002 * r + (rows <= 4096 ? 1.4 * lo + 2.8 * hi : 2.0 * lo + 4.2 * hi);
+  return 1.1 * block / (single - 3.2);
+}
+
 // (Not in a context with a scratch limit: the copy of the sketch that the HBM path permutes, which
 // the register-resident grid does without, would be held when the steps that follow need room.)
 bool lra_qrcp_blocks_fit(lra_ctx* c, int m, int n) {
@@ -1475,11 +1494,6 @@ int lra_qrcp_global(lra_ctx* c, const QrcpCall& q) {
         }
         return LRA_OK;
       };
-      // Blocks of steps where their workspace fits the budget (LRA_QG_BLOCK=0: single steps
-      // only).  A block takes 50 to 88 us (rows 900 to 2056, 3758 columns) against 10 to 24 us
-      // for a single step, about four of them, so where the blocks come out shorter than
-      // kShort steps on average (many columns of nearly equal norm, or norms outside the
-      // blocks' range) single steps run, twice as many each time.
       const char* be = getenv("LRA_QG_BLOCK");
       // In a context with a scratch limit the blocks' workspace (0.1 MB and 128 bytes a row) goes
       // back at the end, so that single steps' limits still hold what follows.
@@ -1492,28 +1506,36 @@ int lra_qrcp_global(lra_ctx* c, const QrcpCall& q) {
       if (!block) {
         LRA_CHECK(single(0, q.kmax));
       } else {
+        // One block, then batches of them while they come out long enough (`block_steps_needed`);
+        // where they do not, single steps run, twice as many each time.  LRA_QG_BLOCK=0: single
+        // steps only, 1: blocks of three steps and more at any size.
         const QbWork w = lra_qb_work(wb, m);
-        constexpr int kBatch = 8, kShort = 3;
-        LRA_CHECK(lra_qb_start(c, q, w, at, vn1, diag, fs));
-        for (int s = 0, run = 64;;) {
-          LRA_CHECK(lra_qb_blocks(c, q, w, at, vn1, vn2, diag, fs, s, kBatch));
-          LRA_CHECK(read_state(&h));
-          const int steps = h.s - s;
-          s = h.s;
-          if (h.done) break;
-          if (steps >= kShort * kBatch) {
-            run = 64;
-            continue;
+        const bool force = be && be[0] == '1';
+        auto needed = [&](int s) { return force ? 3.0 : block_steps_needed(m - s, n - s); };
+        constexpr int kBatch = 8;
+        for (int s = 0, run = 128; s < q.kmax && !h.done; s = h.s) {
+          const int cap = lra_qb_cap(m - s);
+          if (needed(s) > cap) {  // no block here would be worth it: on to where more steps fit one
+            const int top = cap == 4 ? 4096 : cap == 8 ? 3072 : cap == 12 ? 2048 : 0;
+            LRA_CHECK(single(s, m - s - top));
+          } else {
+            LRA_CHECK(lra_qb_start(c, q, w, at, vn1, diag, fs));
+            for (int count = 1;; count = kBatch, run = 128) {
+              const double need = needed(s);
+              LRA_CHECK(lra_qb_blocks(c, q, w, at, vn1, vn2, diag, fs, s, count));
+              LRA_CHECK(read_state(&h));
+              const int steps = h.s - s;
+              s = h.s;
+              if (h.done || steps < need * count || needed(s) > lra_qb_cap(m - s)) break;
+            }
+            if (h.done) break;
+            LRA_CHECK(lra_qb_pick(c, w, at, fs));
+            LRA_CHECK(single(s, run));
+            run = std::min(2 * run, 4096);
           }
-          LRA_CHECK(lra_qb_pick(c, w, at, fs));
-          LRA_CHECK(single(s, run));
           hipLaunchKernelGGL(qg_ffinish, dim3(1), dim3(256), 0, s0, m, q.A, q.lda, at, diag, v, fs,
                              q.k_out, q.early_out);
-          LRA_CHECK(lra_qb_start(c, q, w, at, vn1, diag, fs));
           LRA_CHECK(read_state(&h));
-          s = h.s;
-          if (h.done) break;
-          run = std::min(2 * run, 4096);
         }
       }
       hipLaunchKernelGGL(qg_ffinish, dim3(1), dim3(256), 0, s0, m, q.A, q.lda, at, diag, v, fs,

@@ -257,3 +257,24 @@ def test_blocks_repeat_their_bits(gpu, monkeypatch, m, n):
         assert k == len(ref[1]) and k > 300
         for what, a, b in zip(("pivots", "tau", "factors"), got, ref):
             assert np.array_equal(a, b), (what, np.argwhere(a != b)[:4])
+
+
+@pytest.mark.parametrize("m,n", [(8192, 264), (5000, 520), (4096, 200)])
+def test_tall_sketches_take_single_steps(gpu, monkeypatch, m, n):
+    """Sketches on which a block of steps costs more than the steps it holds (tall, with few columns)
+    run in single steps: the bits of LRA_QG_BLOCK=0."""
+    import torch
+    monkeypatch.setenv("LRA_QRCP_GLOBAL", "1")
+    rng = np.random.default_rng(m)
+    B = (rng.standard_normal((m, n)) * np.exp(-0.01 * np.arange(n))) @ rng.standard_normal((n, n))
+    out = []
+    for block in (None, "0"):
+        if block:
+            monkeypatch.setenv("LRA_QG_BLOCK", block)
+        Bd = gpu.to_device(np.asfortranarray(B))
+        p, tau, k = gpu.geqp3_adap(Bd, 100, 0.0, 0.0, 32)
+        torch.cuda.synchronize()
+        out.append((k, host(p), host(tau)[:k], host(Bd)))
+    assert out[0][0] == out[1][0] == 100
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert np.array_equal(a, b)
