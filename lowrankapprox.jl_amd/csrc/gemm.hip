@@ -1162,17 +1162,25 @@ int run_direct(lra_ctx* ctx, const GemmArgs& g) {
   return LRA_OK;
 }
 
-// A short-K product with a tall C (the blocked QR's X -= V W and its like): in FP64 on
-// gemm_direct_kernel.  The low precisions form the transposed product C' = op(B)' op(A)' stored
-// transposed: the MFMA output tile then puts 16 consecutive rows of one column of C in 16
-// consecutive lanes, so the read-modify-write of C is coalesced.  One K-range, the general
-// kernel's configuration for the swapped shape.
+// A short-K product with a tall C (the blocked QR's X -= V W and its like): formed as the
+// transposed product C' = op(B)' op(A)' stored transposed, so that the MFMA output tile puts 16
+// consecutive rows of one column of C in 16 consecutive lanes and the read-modify-write of C is
+// coalesced.  One K-range, the general kernel's configuration for the swapped shape.
 bool ct_ok(const GemmArgs& g) {
   return g.bgather == nullptr && g.K <= 64 && g.M >= 256 && g.M >= 2 * g.N;
 }
+// In FP64 with more than 32 columns, gemm_direct_kernel takes it (with the same bits) up to 2 M
+// elements of C, where the tiles are few; beyond, only where op(B) is read along its columns or K
+// is short.  Tiled -> direct: 4096 x 512 at K = 64 29 -> 18 to 26 us, 8192 x 2048 at K = 8 68 -> 50,
+// with op(B) = B' at K = 64 108 -> 85, but with op(B) = B at K = 32 82 -> 94 and 16384 x 4096 306 ->
+// 450; 60000 x 16 at K = 64 17 -> 27.
+bool ct_direct(const GemmArgs& g) {
+  return g.prec == LRA_PREC_F64 && g.K >= 1 && g.N > 32 &&
+         (g.M * g.N <= (1ll << 21) || g.transB || (g.K <= 16 && g.M * g.N <= (1ll << 25)));
+}
 
 int run_ct(lra_ctx* ctx, const GemmArgs& g) {
-  if (g.prec == LRA_PREC_F64 && g.K >= 1) return run_direct(ctx, g);
+  if (ct_direct(g)) return run_direct(ctx, g);
   GemmArgs s = g;
   s.M = g.N; s.N = g.M;
   s.A = g.B; s.lda = g.ldb; s.transA = !g.transB;

@@ -377,3 +377,25 @@ def test_choice_of_an_untuned_kernel(gpu):
         return gpu._lib.load().lra_gemm_choice(0, 0, 0, 1000, N, 300, *(ctypes.byref(ctypes.c_int())
                                                                        for _ in range(4)))
     assert choice(4000) == 0 and choice(2060) != 0
+
+
+@pytest.mark.parametrize("ta", ["n", "c"])
+@pytest.mark.parametrize("tb", ["n", "c"])
+@pytest.mark.parametrize("M,N,K,rows,cols", [(900, 33, 17, 900, 32), (300, 40, 64, 300, 7),
+                                             (65700, 33, 32, 63000, 33), (65700, 33, 1, 300, 20),
+                                             (8200, 300, 20, 6000, 300)])
+def test_short_k_products_same_bits(gpu, ta, tb, M, N, K, rows, cols):
+    """A tall product with a short K gives the same bits straight to the MFMAs and on the tiles
+    (rules on the number of columns and elements): a block of its rows and columns, formed alone,
+    against the whole, and the whole against numpy."""
+    rng = np.random.default_rng(M + N + K)
+    A, B, C = rng.standard_normal((M, K)), rng.standard_normal((K, N)), rng.standard_normal((M, N))
+
+    def form(A, B, C):
+        Cd = gpu.to_device(np.asfortranarray(C)).clone().t().contiguous().t()
+        op = lambda X, t: np.asfortranarray(X if t == "n" else X.T)
+        return host(gpu.dgemm(op(A, ta), op(B, tb), ta, tb, -1.25, Cd, 0.75))
+    whole, part = form(A, B, C), form(A[:rows], B[:, :cols], C[:rows, :cols])
+    assert np.array_equal(whole[:rows, :cols], part)
+    bound = 2.3e-16 * (K + 4) * (1.25 * np.abs(A) @ np.abs(B) + np.abs(C))
+    assert (np.abs(whole - (0.75 * C - 1.25 * A @ B)) <= bound).all()
