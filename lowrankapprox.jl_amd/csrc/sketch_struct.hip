@@ -372,10 +372,14 @@ __global__ __launch_bounds__(256) void srft_slots_kernel(
 // 226; at l = 12 of 12108 x 50 they are even, and for a smaller l, where the sums over q are the
 // work, srft_kernel is ahead (l = 9 of 45027 x 3000 3400, two kernels 7200).  Below 4 M complex
 // products the extra launches cost more than they give (200 x 100 at l = 40: 42 and 46, 1000 x
-// 300 at l = 50 64 and 55).
+// 300 at l = 50 64 and 55); below l = 36 that holds for a short column at any number of them that
+// srft_kernel's grid holds at once (l = 20 of 620 x 1000 29 and 38, l = 30 of 930 x 1000 39 and
+// 42, but l = 20 of 160 x 3000 53 and 37, l = 30 of 930 x 3000 85 and 69, and, of 2000 x 100, 61 and 50).
 bool srft_split(i64 l, i64 P, i64 Q) {
   if (const char* e = getenv("LRA_SRFT_SPLIT")) return e[0] != '0';
-  return l >= 16 && (double)l * (double)P * (double)Q >= 4e6;
+  const i64 mm = P / l;
+  return l >= 16 && (double)l * (double)P * (double)Q >= 4e6 &&
+         (l >= 36 || mm >= 64 || (Q >= 2048 && (l >= 24 || mm < 16)));
 }
 
 // LRA_E_ALLOC: no memory for the workspace, and nothing was done.
