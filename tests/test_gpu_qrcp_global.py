@@ -278,3 +278,54 @@ def test_tall_sketches_take_single_steps(gpu, monkeypatch, m, n):
     assert out[0][0] == out[1][0] == 100
     for a, b in zip(out[0][1:], out[1][1:]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("m,n,fall,rtol,env,opts", [
+    (900, 700, 0.03, 1e-7, {"LRA_QRCP_GLOBAL": "1"}, {}),
+    # rounds of 24, 48, ... columns: their stops and dlaqps blocks end inside blocks of 16
+    (900, 800, 0.02, 1e-5, {"LRA_QRCP_GLOBAL": "1"}, {"nb": 24}),
+    (700, 1200, 0.1, 1e-9, {"LRA_QRCP_GLOBAL": "1"}, {"nb": 40}),
+    # orders 520 and 1032 that fit the register-resident grid, foreseen to fall slowly: there in
+    # blocks or (LRA_QG_BLOCK=0) in that grid
+    (1500, 1500, 0.015, 1e-4, {"LRA_QRCP_PAIR": "0"}, {}),
+    (1300, 1900, 0.012, 1e-3, {"LRA_QRCP_PAIR": "0"}, {"nb": 36})])
+@pytest.mark.parametrize("block", ["", "1"])
+def test_blocks_in_adaptive_rounds(gpu, monkeypatch, m, n, fall, rtol, env, opts, block):
+    """An adaptive ID in blocks and in single steps: rounds that are stopped at their target or at the
+    rank inside a block, whose later steps are taken back.  The same rounds, rank, skeleton and order of the
+    redundant columns, T to rounding (relative to its largest entry; R11's condition 1 / rtol)."""
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    rng = np.random.default_rng(m + n)
+    r = min(m, n)
+    U, V = (np.linalg.qr(rng.standard_normal((d, r)))[0] for d in (m, n))
+    A = gpu.to_device((U * np.exp(-fall * np.arange(r))) @ V.T)
+    out = []
+    for b in (block, "0"):
+        monkeypatch.setenv("LRA_QG_BLOCK", b)
+        W = gpu.idfact(A, rtol=rtol, seed=6, **opts)
+        out.append(((W.k, W.rounds), host(W.sk), host(W.rd), host(W.T)))
+    (k1, s1, r1, T1), (k0, s0, r0, T0) = out
+    assert k1 == k0 and k1[0] > 100
+    assert np.array_equal(s1, s0) and np.array_equal(r1, r0)
+    assert np.abs(T1 - T0).max() <= 1e-14 / rtol * np.abs(T0).max()
+
+
+@pytest.mark.parametrize("m,n,fall,rtol", [(2999, 2999, 0.1, 1e-8), (4500, 4200, 0.2, 1e-8),
+                                           (3000, 2500, 0.09, 1e-4), (5000, 4100, 0.03, 1e-3)])
+def test_rounds_alone_and_in_pairs(gpu, monkeypatch, m, n, fall, rtol):
+    """Which rounds share a launch (by size, or alone where a rejected round foresees the next one to
+    be accepted) changes no result: the same ID as with every round alone, T to rounding."""
+    rng = np.random.default_rng(m)
+    r = min(m, n, 400)
+    U, V = (np.linalg.qr(rng.standard_normal((d, r)))[0] for d in (m, n))
+    A = gpu.to_device((U * np.exp(-fall * np.arange(r))) @ V.T)
+    out = []
+    for pair in ("1", "0"):
+        monkeypatch.setenv("LRA_QRCP_PAIR", pair)
+        W = gpu.idfact(A, rtol=rtol, seed=6)
+        out.append(((W.k, W.rounds), host(W.sk), host(W.rd), host(W.T)))
+    (k1, s1, r1, T1), (k0, s0, r0, T0) = out
+    assert k1 == k0 and k1[0] > 32
+    assert np.array_equal(s1, s0) and np.array_equal(r1, r0)
+    assert np.abs(T1 - T0).max() <= 1e-13 / rtol * np.abs(T0).max()
