@@ -1169,14 +1169,16 @@ int run_direct(lra_ctx* ctx, const GemmArgs& g) {
 bool ct_ok(const GemmArgs& g) {
   return g.bgather == nullptr && g.K <= 64 && g.M >= 256 && g.M >= 2 * g.N;
 }
-// In FP64 with more than 32 columns, gemm_direct_kernel takes it (with the same bits) up to 2 M
-// elements of C, where the tiles are few; beyond, only where op(B) is read along its columns or K
-// is short.  Tiled -> direct: 4096 x 512 at K = 64 29 -> 18 to 26 us, 8192 x 2048 at K = 8 68 -> 50,
-// with op(B) = B' at K = 64 108 -> 85, but with op(B) = B at K = 32 82 -> 94 and 16384 x 4096 306 ->
-// 450; 60000 x 16 at K = 64 17 -> 27.
+// In FP64 gemm_direct_kernel takes it (with the same bits) up to 2 M elements of C, where the tiles
+// are few; beyond, only where op(B) is read along its columns or K is short; and with at most 32
+// columns, half its tile or more idle, up to 32768 rows.  Tiled -> direct: 5689 x 16 at K = 32
+// 9.2 -> 6.3 us, 4096 x 512 at K = 64 29 -> 18 to 26, 8192 x 2048 at K = 8 68 -> 50, with op(B) = B'
+// at K = 64 108 -> 85, but with op(B) = B at K = 32 82 -> 94 and 16384 x 4096 306 -> 450; 30000 x 32
+// at K = 32 13.5 -> 10.7, 60000 x 32 14.7 -> 18.8 and x 16 10.0 -> 15.3.
 bool ct_direct(const GemmArgs& g) {
-  return g.prec == LRA_PREC_F64 && g.K >= 1 && g.N > 32 &&
-         (g.M * g.N <= (1ll << 21) || g.transB || (g.K <= 16 && g.M * g.N <= (1ll << 25)));
+  if (g.prec != LRA_PREC_F64 || g.K < 1) return false;
+  if (g.N <= 32) return g.M <= 32768;
+  return g.M * g.N <= (1ll << 21) || g.transB || (g.K <= 16 && g.M * g.N <= (1ll << 25));
 }
 
 int run_ct(lra_ctx* ctx, const GemmArgs& g) {

@@ -383,6 +383,7 @@ def test_choice_of_an_untuned_kernel(gpu):
 @pytest.mark.parametrize("tb", ["n", "c"])
 @pytest.mark.parametrize("M,N,K,rows,cols", [(900, 33, 17, 900, 32), (300, 40, 64, 300, 7),
                                              (65700, 33, 32, 63000, 33), (65700, 33, 1, 300, 20),
+                                             (33000, 9, 33, 30000, 9),
                                              (8200, 300, 20, 6000, 300)])
 def test_short_k_products_same_bits(gpu, ta, tb, M, N, K, rows, cols):
     """A tall product with a short K gives the same bits straight to the MFMAs and on the tiles
