@@ -414,7 +414,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_kc_f64_kernel(Gem
   // waits for this wave's LDS operations, not for its global loads
   auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-  // (the pointer alignment of the 16-byte loads: lda, ldb, kbeg and c are even)
+  // (kbeg and c are even: a pair is on 16 bytes where its column is, else on 8)
   const int full = kbeg < kend ? (kend - kbeg) / BK : 0;
   int cur = 0;
   if (full > 0) {

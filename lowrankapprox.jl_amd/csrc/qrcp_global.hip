@@ -3,8 +3,8 @@
 // kernel of qrcp.hip (e.g. order 1032 or 2056 on thousands of columns).
 //
 // The sketch stays in HBM (column-major, in place).  Up to 8192 rows (with the uncached
-// exchange area) the steps run in blocks of up to 16 (qrcp_block.hip), and where blocks come out
-// short each step is ONE launch, `qg_fused` (below): every workgroup rebuilds the step's
+// exchange area) the steps run in blocks of up to 16 (qrcp_block.hip), and where a block costs more
+// than the steps it holds (`block_steps_needed`) each step is ONE launch, `qg_fused` (below): every workgroup rebuilds the step's
 // reflector itself, and the workgroup that finishes last picks the next pivot.
 // Otherwise (or with LRA_QG_FUSED=0) each step is two launches on the context's stream, with
 // every decision kept on the device:
